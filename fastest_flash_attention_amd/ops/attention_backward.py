@@ -16,7 +16,6 @@ not change the gradients, so it is accepted and ignored.
 
 from __future__ import annotations
 
-import ctypes
 import math
 from typing import Optional, Tuple
 
@@ -144,10 +143,7 @@ def fastest_flash_attn_backward(
         a.softcap = float(softcap) if softcap is not None else 0.0
         a.dtype = code
         a.v_head_dim = Dv if narrow_v else 0
-        stream = _lib.current_stream_handle(dev)
-        with torch.cuda.device(dev):
-            rc = lib.ffa_attn_bwd(ctypes.byref(a), ctypes.c_void_p(stream))
-        _lib.check(rc)
+        _lib.launch(lib.ffa_attn_bwd, a, dev)
     if d_pad != D:
         dq, dk = (t[..., :D].contiguous() for t in (dq, dk))
     if dv.size(-1) != Dv:

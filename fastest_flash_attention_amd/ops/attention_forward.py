@@ -313,11 +313,7 @@ def prepare_prefill(*args, out: Optional[torch.Tensor] = None, **kwargs) -> Pref
 
 
 def launch_prefill(call: PrefillCall) -> None:
-    lib = _lib.load()
-    stream = _lib.current_stream_handle(call.q.device)
-    with torch.cuda.device(call.q.device):
-        rc = lib.ffa_prefill_fwd(ctypes.byref(call.args), ctypes.c_void_p(stream))
-    _lib.check(rc)
+    _lib.launch(_lib.load().ffa_prefill_fwd, call.args, call.q.device)
 
 
 def fastest_flash_attn_forward(

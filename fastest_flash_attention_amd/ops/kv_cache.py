@@ -25,7 +25,6 @@ device reduction and a host sync.
 
 from __future__ import annotations
 
-import ctypes
 import math
 from typing import Optional, Sequence, Tuple
 
@@ -83,7 +82,6 @@ def _paged_decode_fp32(q3, k_pages, v_pages, block_tables, context_lens, scale, 
     lse = (torch.full((B, Hq), float("-inf"), dtype=torch.float32, device=q3.device)
            if return_lse else None)
     lib = _lib.load()
-    stream = _lib.current_stream_handle(q3.device)
     for b, L in enumerate(lens):
         if L == 0:
             continue
@@ -101,8 +99,7 @@ def _paged_decode_fp32(q3, k_pages, v_pages, block_tables, context_lens, scale, 
         g.head_dim = D
         g.context_len = L
         g.elem_bytes = 4
-        with torch.cuda.device(q3.device):
-            _lib.check(lib.ffa_paged_gather(ctypes.byref(g), ctypes.c_void_p(stream)))
+        _lib.launch(lib.ffa_paged_gather, g, q3.device)
         call = prepare_prefill(q3[b, :, None, :].unsqueeze(0), k.unsqueeze(0), v.unsqueeze(0),
                                scale=scale, causal=True, softcap=softcap,
                                sliding_window=sliding_window, num_kv_heads=Hkv,
@@ -258,10 +255,7 @@ def fastest_flash_paged_decode(
     a.scale = float(scale)
     a.softcap = float(softcap) if softcap is not None else 0.0
     a.dtype = code
-    stream = _lib.current_stream_handle(q3.device)
-    with torch.cuda.device(q3.device):
-        rc = lib.ffa_paged_decode_fwd(ctypes.byref(a), ctypes.c_void_p(stream))
-    _lib.check(rc)
+    _lib.launch(lib.ffa_paged_decode_fwd, a, q3.device)
     if not squeeze:
         out = out.unsqueeze(2)
         if lse is not None:
@@ -446,10 +440,7 @@ class PagedKVCache:
         a.elem_bytes = self.k_pages.element_size()
         if a.elem_bytes not in (2, 4):
             raise TypeError(f"PagedKVCache: pool dtype {self.k_pages.dtype} is not supported on the GPU")
-        lib = _lib.load()
-        with torch.cuda.device(self.k_pages.device):
-            stream = _lib.current_stream_handle(self.k_pages.device)
-            _lib.check(lib.ffa_paged_append(ctypes.byref(a), ctypes.c_void_p(stream)))
+        _lib.launch(_lib.load().ffa_paged_append, a, self.k_pages.device)
 
     def _page_table_tensor(self, seq_id: int) -> torch.Tensor:
         return torch.tensor(self.sequences[seq_id]["page_table"], dtype=torch.int32,
@@ -498,11 +489,7 @@ class PagedKVCache:
         a.head_dim = self.head_dim
         a.context_len = L
         a.elem_bytes = self.k_pages.element_size()
-        lib = _lib.load()
-        stream = _lib.current_stream_handle(self.k_pages.device)
-        with torch.cuda.device(self.k_pages.device):
-            rc = lib.ffa_paged_gather(ctypes.byref(a), ctypes.c_void_p(stream))
-        _lib.check(rc)
+        _lib.launch(_lib.load().ffa_paged_gather, a, self.k_pages.device)
         return k_out, v_out
 
     def block_tables(

@@ -18,7 +18,6 @@ projections are torch batched GEMMs.
 
 from __future__ import annotations
 
-import ctypes
 import math
 from dataclasses import dataclass
 from typing import Optional, Sequence, Tuple
@@ -165,11 +164,7 @@ def prepare_mla_decode(
 
 
 def launch_mla_decode(call: MlaDecodeCall) -> None:
-    lib = _lib.load()
-    stream = _lib.current_stream_handle(call.q.device)
-    with torch.cuda.device(call.q.device):
-        rc = lib.ffa_mla_decode_fwd(ctypes.byref(call.args), ctypes.c_void_p(stream))
-    _lib.check(rc)
+    _lib.launch(_lib.load().ffa_mla_decode_fwd, call.args, call.q.device)
 
 
 def fastest_flash_mla_decode(
@@ -298,10 +293,7 @@ class MLALatentCache:
         a.elem_bytes = self.pages.element_size()
         if a.elem_bytes not in (2, 4):
             raise TypeError(f"MLALatentCache: pool dtype {self.pages.dtype} is not supported")
-        lib = _lib.load()
-        with torch.cuda.device(self.pages.device):
-            stream = _lib.current_stream_handle(self.pages.device)
-            _lib.check(lib.ffa_paged_append(ctypes.byref(a), ctypes.c_void_p(stream)))
+        _lib.launch(_lib.load().ffa_paged_append, a, self.pages.device)
 
     def block_tables(self, seq_ids: Sequence[int],
                      device: Optional[torch.device | str] = None
