@@ -20,11 +20,12 @@ import torch  # noqa: F401  (must load torch's HIP runtime before libffa.so)
 
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libffa.so")
 
-FFA_ABI_VERSION = 7
+FFA_ABI_VERSION = 8
 FFA_DTYPE_BF16 = 0
 FFA_DTYPE_FP16 = 1
 FFA_DTYPE_FP32 = 2
 FFA_NOALLOC_SCRATCH_BYTES = 64 << 20  # include/ffa.h
+FFA_SPLIT_MIN_KEYS = 2048  # include/ffa.h
 
 _I64x4 = ctypes.c_int64 * 4
 _I64x3 = ctypes.c_int64 * 3
@@ -64,6 +65,13 @@ class PrefillArgs(ctypes.Structure):
         ("block_key_mask_words", ctypes.c_int32),
         ("block_visited", ctypes.c_void_p),
         ("v_head_dim", ctypes.c_int32),
+        ("k_cache", ctypes.c_void_p),
+        ("v_cache", ctypes.c_void_p),
+        ("k_cache_stride", _I64x4),
+        ("v_cache_stride", _I64x4),
+        ("cache_len", ctypes.c_int32),
+        ("workspace", ctypes.c_void_p),
+        ("workspace_bytes", ctypes.c_size_t),
     ]
 
 
@@ -210,6 +218,7 @@ class AttnBwdArgs(ctypes.Structure):
 # Every symbol include/ffa.h declares, with its ctypes signature.
 EXPORTS = {
     "ffa_prefill_fwd": (ctypes.c_int, [ctypes.POINTER(PrefillArgs), ctypes.c_void_p]),
+    "ffa_prefill_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(PrefillArgs)]),
     "ffa_paged_gather": (ctypes.c_int, [ctypes.POINTER(PagedGatherArgs), ctypes.c_void_p]),
     "ffa_paged_append": (ctypes.c_int, [ctypes.POINTER(PagedAppendArgs), ctypes.c_void_p]),
     "ffa_paged_decode_num_splits": (ctypes.c_int32, [ctypes.c_int32, ctypes.c_int32]),

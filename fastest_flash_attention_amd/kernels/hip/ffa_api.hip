@@ -71,6 +71,86 @@ int check_decode_args(const ffa_paged_decode_args* a, bool* empty) {
   return FFA_OK;
 }
 
+// Every check of a prefill call. *empty: nothing to launch.
+int check_prefill_args(const ffa_prefill_args* a, bool* empty) {
+  *empty = false;
+  if (a == nullptr) return FFA_ERR_INVALID_ARG;
+  if (!valid_dtype(a->dtype) && a->dtype != FFA_DTYPE_FP32) return FFA_ERR_UNSUPPORTED_DTYPE;
+  if (a->head_dim < 1 || a->head_dim > 256) return FFA_ERR_UNSUPPORTED_HEAD_DIM;
+  if (const int rc = check_v_head_dim(a->v_head_dim, a->head_dim, a->dtype); rc != FFA_OK) return rc;
+  if (a->batch < 0 || a->heads_q < 1 || a->heads_kv < 1 || a->seqlen_q < 0 || a->seqlen_kv < 0) {
+    return FFA_ERR_INVALID_ARG;
+  }
+  if (a->heads_q % a->heads_kv != 0) return FFA_ERR_GQA_RATIO;
+  const bool cached = a->k_cache != nullptr;
+  if (cached && (a->cache_len < 0 || a->cache_len > a->seqlen_kv || a->v_cache == nullptr)) {
+    return FFA_ERR_INVALID_ARG;
+  }
+  if (a->batch == 0 || a->seqlen_q == 0) {
+    *empty = true;
+    return FFA_OK;
+  }
+  if (a->q == nullptr || a->o == nullptr) return FFA_ERR_INVALID_ARG;
+  if (a->seqlen_kv > (cached ? a->cache_len : 0) && (a->k == nullptr || a->v == nullptr)) {
+    return FFA_ERR_INVALID_ARG;
+  }
+  if (a->q_stride[3] != 1 || a->k_stride[3] != 1 || a->v_stride[3] != 1 || a->o_stride[3] != 1) {
+    return FFA_ERR_INVALID_ARG;
+  }
+  for (int i = 0; i < 3; ++i) {
+    if (a->q_stride[i] < 0 || a->k_stride[i] < 0 || a->v_stride[i] < 0 || a->o_stride[i] < 0 ||
+        a->lse_stride[i] < 0) {
+      return FFA_ERR_INVALID_ARG;
+    }
+  }
+  if (!valid_scale(a->scale, a->softcap)) return FFA_ERR_INVALID_ARG;
+  if (cached) {
+    if (a->k_cache_stride[3] != 1 || a->v_cache_stride[3] != 1) return FFA_ERR_INVALID_ARG;
+    for (int i = 0; i < 3; ++i) {
+      if (a->k_cache_stride[i] < 0 || a->v_cache_stride[i] < 0) return FFA_ERR_INVALID_ARG;
+    }
+  }
+  // 16-byte vector / direct-to-LDS loads: aligned bases, head_dim and row strides in
+  // whole 16-byte chunks.
+  if (a->head_dim % 8 != 0) return FFA_ERR_MISALIGNED;
+  const void* ptrs[7] = {a->q, a->k, a->v, a->o, a->workspace, a->k_cache, a->v_cache};
+  for (const void* ptr : ptrs) {
+    if ((reinterpret_cast<uintptr_t>(ptr) & 15u) != 0) return FFA_ERR_MISALIGNED;
+  }
+  const int64_t* strides[4] = {a->q_stride, a->k_stride, a->v_stride, a->o_stride};
+  for (const int64_t* st : strides) {
+    for (int i = 0; i < 3; ++i) {
+      if (st[i] % 8 != 0) return FFA_ERR_MISALIGNED;
+    }
+  }
+  if (cached) {
+    for (int i = 0; i < 3; ++i) {
+      if (a->k_cache_stride[i] % 8 != 0 || a->v_cache_stride[i] % 8 != 0) return FFA_ERR_MISALIGNED;
+    }
+  }
+  if (a->block_key_mask != nullptr) {
+    const int64_t need_words = (static_cast<int64_t>(a->seqlen_kv) + 63) / 64;
+    if (a->block_visited == nullptr || a->block_key_mask_words < need_words ||
+        a->ref_block_q <= 0 || (reinterpret_cast<uintptr_t>(a->block_key_mask) & 7u) != 0) {
+      return FFA_ERR_INVALID_ARG;
+    }
+  }
+  // per-tile byte offsets of K/V rows are 32-bit
+  if (a->k_stride[2] >= (int64_t{1} << 24) || a->v_stride[2] >= (int64_t{1} << 24)) {
+    return FFA_ERR_TOO_LARGE;
+  }
+  if (cached &&
+      (a->k_cache_stride[2] >= (int64_t{1} << 24) || a->v_cache_stride[2] >= (int64_t{1} << 24))) {
+    return FFA_ERR_TOO_LARGE;
+  }
+  // Positions are int32 inside the kernel.
+  const int64_t max_pos = static_cast<int64_t>(a->q_offset) + a->seqlen_q;
+  if (max_pos > ffa::kMaxPos || a->seqlen_kv > ffa::kMaxPos || a->q_offset < -ffa::kMaxPos) {
+    return FFA_ERR_TOO_LARGE;
+  }
+  return FFA_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -111,57 +191,19 @@ const char* ffa_strerror(int status) {
 }
 
 int ffa_prefill_fwd(const ffa_prefill_args* a, void* stream) {
-  if (a == nullptr) return FFA_ERR_INVALID_ARG;
-  if (!valid_dtype(a->dtype) && a->dtype != FFA_DTYPE_FP32) return FFA_ERR_UNSUPPORTED_DTYPE;
-  if (a->head_dim < 1 || a->head_dim > 256) return FFA_ERR_UNSUPPORTED_HEAD_DIM;
-  if (const int rc = check_v_head_dim(a->v_head_dim, a->head_dim, a->dtype); rc != FFA_OK) return rc;
-  if (a->batch < 0 || a->heads_q < 1 || a->heads_kv < 1 || a->seqlen_q < 0 || a->seqlen_kv < 0) {
-    return FFA_ERR_INVALID_ARG;
-  }
-  if (a->heads_q % a->heads_kv != 0) return FFA_ERR_GQA_RATIO;
-  if (a->batch == 0 || a->seqlen_q == 0) return FFA_OK;
-  if (a->q == nullptr || a->o == nullptr) return FFA_ERR_INVALID_ARG;
-  if (a->seqlen_kv > 0 && (a->k == nullptr || a->v == nullptr)) return FFA_ERR_INVALID_ARG;
-  if (a->q_stride[3] != 1 || a->k_stride[3] != 1 || a->v_stride[3] != 1 || a->o_stride[3] != 1) {
-    return FFA_ERR_INVALID_ARG;
-  }
-  for (int i = 0; i < 3; ++i) {
-    if (a->q_stride[i] < 0 || a->k_stride[i] < 0 || a->v_stride[i] < 0 || a->o_stride[i] < 0 ||
-        a->lse_stride[i] < 0) {
-      return FFA_ERR_INVALID_ARG;
-    }
-  }
-  if (!valid_scale(a->scale, a->softcap)) return FFA_ERR_INVALID_ARG;
-  // 16-byte vector / direct-to-LDS loads: aligned bases, head_dim and row strides in
-  // whole 16-byte chunks.
-  if (a->head_dim % 8 != 0) return FFA_ERR_MISALIGNED;
-  const void* ptrs[4] = {a->q, a->k, a->v, a->o};
-  for (const void* ptr : ptrs) {
-    if ((reinterpret_cast<uintptr_t>(ptr) & 15u) != 0) return FFA_ERR_MISALIGNED;
-  }
-  const int64_t* strides[4] = {a->q_stride, a->k_stride, a->v_stride, a->o_stride};
-  for (const int64_t* st : strides) {
-    for (int i = 0; i < 3; ++i) {
-      if (st[i] % 8 != 0) return FFA_ERR_MISALIGNED;
-    }
-  }
-  if (a->block_key_mask != nullptr) {
-    const int64_t need_words = (static_cast<int64_t>(a->seqlen_kv) + 63) / 64;
-    if (a->block_visited == nullptr || a->block_key_mask_words < need_words ||
-        a->ref_block_q <= 0 || (reinterpret_cast<uintptr_t>(a->block_key_mask) & 7u) != 0) {
-      return FFA_ERR_INVALID_ARG;
-    }
-  }
-  // per-tile byte offsets of K/V rows are 32-bit
-  if (a->k_stride[2] >= (int64_t{1} << 24) || a->v_stride[2] >= (int64_t{1} << 24)) {
-    return FFA_ERR_TOO_LARGE;
-  }
-  // Positions are int32 inside the kernel.
-  const int64_t max_pos = static_cast<int64_t>(a->q_offset) + a->seqlen_q;
-  if (max_pos > ffa::kMaxPos || a->seqlen_kv > ffa::kMaxPos || a->q_offset < -ffa::kMaxPos) {
-    return FFA_ERR_TOO_LARGE;
-  }
+  bool empty = false;
+  const int rc = check_prefill_args(a, &empty);
+  if (rc != FFA_OK || empty) return rc;
   return ffa::launch_prefill(*a, static_cast<hipStream_t>(stream));
+}
+
+size_t ffa_prefill_workspace_bytes(const ffa_prefill_args* a) {
+  if (a == nullptr || a->batch < 0 || a->heads_q < 1 || a->heads_kv < 1 ||
+      a->heads_q % a->heads_kv != 0 || a->seqlen_q < 0 || a->seqlen_kv < 0 || a->head_dim < 1 ||
+      a->head_dim > 256 || (a->k_cache != nullptr && (a->cache_len < 0 || a->cache_len > a->seqlen_kv))) {
+    return 0;
+  }
+  return ffa::prefill_workspace_bytes(*a);
 }
 
 int ffa_paged_gather(const ffa_paged_gather_args* a, void* stream) {

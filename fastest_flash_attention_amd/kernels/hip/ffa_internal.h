@@ -8,7 +8,9 @@
 
 namespace ffa {
 
-// Prefill: one launch of the fused forward kernel.
+// Prefill: one launch of the fused forward kernel, or (few rows over many keys, with a
+// workspace) the split kernel and its merge.
+size_t prefill_workspace_bytes(const ffa_prefill_args& a);
 int launch_prefill(const ffa_prefill_args& a, hipStream_t stream);
 
 // Paged decode: split kernel + logsumexp combine kernel.

@@ -94,8 +94,17 @@ constexpr int kMinBlocks = (DP == 64 && !SOFTCAP) ? 3 : (DP <= 192 ? 2 : 1);
 // (B 2, H 32, S 4096): +4-6 % causal, +5 % non-causal, +-0-2 % with softcap, outputs
 // bit-identical, and the kernel stops spilling; the head_dim-128 kernels lose 3-8 %
 // with eight waves, and shorter causal sequences lose too (-10 % at S = 2048).
+// SPLIT (Tag = SplitKeys<...>): few query rows over many keys (a new token or a chunk over
+// a KV cache, a short prompt of a small model). One workgroup per 128 rows of a head
+// leaves most of the chip idle there, so the keys are split too: workgroups = (batch, KV
+// head) x key ranges x query tiles, each leaving a partial result for
+// prefill_merge_kernel. The rows of a group's query heads share tiles when that needs
+// fewer of them (sp.pack), and the cached keys are read where they lie, so a call with a
+// cache needs no concatenated copy of it.
 template <typename Tag, int DP, int DV, int BN, bool SOFTCAP, int NW>
 __global__ __launch_bounds__((64 * NW), (kMinBlocks<DP, SOFTCAP> * 4 / NW)) void prefill_kernel(const PrefillParams p) {
+  constexpr bool SPLIT = kSplitKeys<Tag>;
+  const SplitParams& sp = p.sp;
   constexpr int BM = 32 * NW;  // query rows per workgroup
   using S = Shape<DP, BN, NW>;   // Q, K tiles, S^T
   using SV = Shape<DV, BN, NW>;  // V tiles, O^T
@@ -114,39 +123,91 @@ __global__ __launch_bounds__((64 * NW), (kMinBlocks<DP, SOFTCAP> * 4 / NW)) void
   const int l32 = lane & 31;
   const int g = lane >> 5;
 
-  int bh, jq;
-  work_item(p, blockIdx.x, bh, jq);
-  bh = __builtin_amdgcn_readfirstlane(bh);  // uniform: keeps the tile bases in SGPRs
-  jq = __builtin_amdgcn_readfirstlane(jq);
-  const int qt = p.causal ? (p.n_qt - 1 - jq) : jq;
-  const int b = bh / p.Hq;
-  const int h = bh - b * p.Hq;
-  const int hk = h / p.ratio;
+  int b, h, hk, qt;
+  int q_offset = p.q_offset;
+  int Skv = p.Skv;
+  int n_rows = p.Sq;   // rows of this unit's query tiles
+  int kv_first = 0;    // SPLIT: first key of the workgroup's range
+  int split = 0;
+  const uint16_t* kseg = p.k;
+  const uint16_t* vseg = p.v;
+  int64_t k_sb = p.k_sb, k_sh = p.k_sh, k_ss = p.k_ss;
+  int64_t v_sb = p.v_sb, v_sh = p.v_sh, v_ss = p.v_ss;
+  if constexpr (!SPLIT) {
+    int bh, jq;
+    work_item(p, blockIdx.x, bh, jq);
+    bh = __builtin_amdgcn_readfirstlane(bh);  // uniform: keeps the tile bases in SGPRs
+    jq = __builtin_amdgcn_readfirstlane(jq);
+    qt = p.causal ? (p.n_qt - 1 - jq) : jq;
+    b = bh / p.Hq;
+    h = bh - b * p.Hq;
+    hk = h / p.ratio;
+  } else {
+    // The workgroups that read one key range (a KV head's query heads and query tiles)
+    // have consecutive ids on one XCD, so the range comes from HBM once.
+    int id = blockIdx.x;
+    if (p.xcd_remap) id = (id & 7) * (static_cast<int>(gridDim.x) >> 3) + (id >> 3);
+    id = __builtin_amdgcn_readfirstlane(id);
+    const int heads = sp.pack ? 1 : p.ratio;  // units per KV head
+    const int per = heads * p.n_qt;
+    const int range = id / per;
+    const int in = id - range * per;
+    const int hl = in / p.n_qt;
+    qt = p.n_qt - 1 - (in - hl * p.n_qt);
+    split = range % sp.n_split;
+    const int bk = range / sp.n_split;
+    b = bk / p.Hkv;
+    hk = bk - b * p.Hkv;
+    h = hk * p.ratio + hl;
+    if (sp.pack) n_rows = p.Sq * p.ratio;
+    // Key positions become relative to the segment the range lies in (kv_first is a
+    // multiple of BN in it): the cached keys, then the call's own.
+    if (split < sp.n0) {
+      kseg = sp.kc;
+      vseg = sp.vc;
+      k_sb = sp.kc_sb, k_sh = sp.kc_sh, k_ss = sp.kc_ss;
+      v_sb = sp.vc_sb, v_sh = sp.vc_sh, v_ss = sp.vc_ss;
+      kv_first = sp.lo0 + split * sp.len;
+      Skv = min(kv_first + sp.len, sp.cache_len);
+    } else {
+      q_offset -= sp.cache_len;
+      kv_first = sp.lo1 + (split - sp.n0) * sp.len;
+      Skv = min(kv_first + sp.len, p.Skv - sp.cache_len);
+    }
+  }
 
   const uint16_t* __restrict__ qbase = p.q + b * p.q_sb + h * p.q_sh;
-  const char* kbytes = reinterpret_cast<const char*>(p.k + b * p.k_sb + hk * p.k_sh);
-  const char* vbytes = reinterpret_cast<const char*>(p.v + b * p.v_sb + hk * p.v_sh);
+  const char* kbytes = reinterpret_cast<const char*>(kseg + b * k_sb + hk * k_sh);
+  const char* vbytes = reinterpret_cast<const char*>(vseg + b * v_sb + hk * v_sh);
   const int D = p.D;
-  const int Skv = p.Skv;
 
   const int q0 = qt * BM;
-  const int q_last = min(q0 + BM, p.Sq) - 1;
-  const int q0_abs = p.q_offset + q0;
-  const int ql_abs = p.q_offset + q_last;
-  const int kv_lo = p.window > 0 ? max(0, q0_abs - p.window + 1) : 0;
+  const int q_last = min(q0 + BM, n_rows) - 1;
+  // Packed rows (SPLIT): row r is query r % Sq of the group's head r / Sq, so every
+  // workgroup and wave takes the whole range of query positions as its bounds.
+  const bool pack = SPLIT && sp.pack;
+  const int q0_abs = pack ? q_offset : q_offset + q0;
+  const int ql_abs = pack ? q_offset + p.Sq - 1 : q_offset + q_last;
+  const int kv_lo = max(SPLIT ? kv_first : 0, p.window > 0 ? max(0, q0_abs - p.window + 1) : 0);
   const int kv_hi = p.causal ? min(Skv, ql_abs + 1) : Skv;
   const int t_begin = kv_lo / BN;
   const int nt = kv_hi > kv_lo ? (kv_hi + BN - 1) / BN - t_begin : 0;
 
   const int qw0 = q0 + wave * 32;
-  const int qrow = qw0 + l32;
-  const bool wave_live = qw0 < p.Sq;
-  const int qw0_abs = p.q_offset + qw0;
-  const int qwl_abs = p.q_offset + min(qw0 + 31, p.Sq - 1);
-  const int qa = p.q_offset + qrow;
+  int qrow = qw0 + l32;      // this lane's query row, and its head's offset from h (packed)
+  int qhead = 0;
+  const bool wave_live = qw0 < n_rows;
+  if (pack) {
+    qhead = min(qrow, n_rows - 1) / p.Sq;
+    qrow = min(qrow, n_rows - 1) - qhead * p.Sq;
+  }
+  const int qw0_abs = pack ? q0_abs : q_offset + qw0;
+  const int qwl_abs = pack ? ql_abs : q_offset + min(qw0 + 31, p.Sq - 1);
+  const int qa = q_offset + qrow;
   // block mask: this lane's row block in the expanded key mask
+  const uint64_t* const kmask = p.kmask;  // (a split call has no cached keys with one)
   const uint64_t* kmask_row =
-      p.kmask != nullptr ? p.kmask + static_cast<int64_t>(min(qrow, p.Sq - 1) / p.ref_bq) * p.kmask_words
+      kmask != nullptr ? kmask + static_cast<int64_t>(min(qrow, p.Sq - 1) / p.ref_bq) * p.kmask_words
                          : nullptr;
 
   // Block mask: list the tiles of [t_begin, t_begin + nt) whose keys have any set bit
@@ -154,11 +215,11 @@ __global__ __launch_bounds__((64 * NW), (kMinBlocks<DP, SOFTCAP> * 4 / NW)) void
   // blocks rb0 .. rb1). A tile without one contributes nothing (every score is masked),
   // so skipping it changes no result; the fully-masked-row LSE comes from the
   // reference's visited-tile counts, not from the tiles this kernel visits.
-  const bool use_list = p.kmask != nullptr && nt <= kMaxLiveTiles;
+  const bool use_list = kmask != nullptr && nt <= kMaxLiveTiles;
   int n_it = nt;  // iterations of the sweep: nt, or the live tiles with a block mask
   if (use_list) {
-    const int rb0 = q0 / p.ref_bq;
-    const int rb1 = q_last / p.ref_bq;
+    const int rb0 = (pack ? 0 : q0) / p.ref_bq;
+    const int rb1 = (pack ? p.Sq - 1 : q_last) / p.ref_bq;
     int n_live = 0;
     for (int base = 0; base < nt; base += 64 * NW) {
       const int i = base + tid;
@@ -168,7 +229,7 @@ __global__ __launch_bounds__((64 * NW), (kMinBlocks<DP, SOFTCAP> * 4 / NW)) void
         const int kt0 = (t_begin + i) * BN;
         const uint64_t all = BN < 64 ? (uint64_t{1} << (BN & 63)) - 1 : ~uint64_t{0};
         for (int rb = rb0; rb <= rb1; ++rb) {
-          uint64_t w = p.kmask[static_cast<int64_t>(rb) * p.kmask_words + (kt0 >> 6)];
+          uint64_t w = kmask[static_cast<int64_t>(rb) * p.kmask_words + (kt0 >> 6)];
           if constexpr (BN < 64) w = (w >> (kt0 & 63)) & all;
           live = live || w != 0;
           full = full && w == all;
@@ -194,7 +255,7 @@ __global__ __launch_bounds__((64 * NW), (kMinBlocks<DP, SOFTCAP> * 4 / NW)) void
   };
   // whether the block mask needs element tests on sweep position i
   auto kmask_partial = [&](int i) {
-    return p.kmask != nullptr && !(use_list && (live_lds[i] & kTileFull));
+    return kmask != nullptr && !(use_list && (live_lds[i] & kTileFull));
   };
 
   // Scores stay in raw units until the exponent: p = exp2(s*c - m*c), with s = q.k and
@@ -217,7 +278,7 @@ __global__ __launch_bounds__((64 * NW), (kMinBlocks<DP, SOFTCAP> * 4 / NW)) void
     const int row = pos / S::CPR;
     const int q = pos - row * S::CPR;
     const int kc = min(q ^ kswz<DP>(row), dchunks - 1);
-    k_off[j] = static_cast<uint32_t>(row * p.k_ss * 2 + kc * 16);
+    k_off[j] = static_cast<uint32_t>(row * k_ss * 2 + kc * 16);
   }
 #pragma unroll
   for (int j = 0; j < SV::LPT; ++j) {
@@ -225,15 +286,15 @@ __global__ __launch_bounds__((64 * NW), (kMinBlocks<DP, SOFTCAP> * 4 / NW)) void
     const int row = pos / SV::CPR;
     const int q = pos - row * SV::CPR;
     const int vc = min(q ^ vswz<DV>(row), dvchunks - 1);
-    v_off[j] = static_cast<uint32_t>(row * p.v_ss * 2 + vc * 16);
+    v_off[j] = static_cast<uint32_t>(row * v_ss * 2 + vc * 16);
   }
   // The loads are issued from inline asm (wave-uniform tile base + 32-bit lane offset):
   // the compiler neither holds a 64-bit address per load nor guards later LDS reads
   // with vmcnt waits; completion is the explicit wait_vmcnt0 before each tile barrier.
   // K and V tiles are issued in order, so each tensor keeps a running tile base that
   // advances by one tile per issue (one 64-bit scalar add per tile).
-  const int64_t k_tile_bytes = static_cast<int64_t>(BN) * p.k_ss * 2;
-  const int64_t v_tile_bytes = static_cast<int64_t>(BN) * p.v_ss * 2;
+  const int64_t k_tile_bytes = static_cast<int64_t>(BN) * k_ss * 2;
+  const int64_t v_tile_bytes = static_cast<int64_t>(BN) * v_ss * 2;
   const int t_full = Skv / BN;  // tiles below this index hold BN keys
   auto issue_tile = [&](auto shp, const char*& tb, int64_t tile_bytes, int64_t stride,
                         const auto& off, uint16_t* dst, int t) __attribute__((always_inline)) {
@@ -277,11 +338,11 @@ __global__ __launch_bounds__((64 * NW), (kMinBlocks<DP, SOFTCAP> * 4 / NW)) void
   // list can jump, so there the pointer is set from t first.
   auto issue_k = [&](int t, uint16_t* dst) __attribute__((always_inline)) {
     if (use_list) k_next = kbytes + static_cast<int64_t>(t) * k_tile_bytes;
-    issue_tile(S{}, k_next, k_tile_bytes, p.k_ss, k_off, dst, t);
+    issue_tile(S{}, k_next, k_tile_bytes, k_ss, k_off, dst, t);
   };
   auto issue_v = [&](int t, uint16_t* dst) __attribute__((always_inline)) {
     if (use_list) v_next = vbytes + static_cast<int64_t>(t) * v_tile_bytes;
-    issue_tile(SV{}, v_next, v_tile_bytes, p.v_ss, v_off, dst, t);
+    issue_tile(SV{}, v_next, v_tile_bytes, v_ss, v_off, dst, t);
   };
 
   // ---- per-lane LDS operand addresses (element offsets inside one tile buffer) ----
@@ -315,7 +376,7 @@ __global__ __launch_bounds__((64 * NW), (kMinBlocks<DP, SOFTCAP> * 4 / NW)) void
   // retire in issue order). On MI355X: -1 round trip of start-up per workgroup.
   u32x4 qreg[S::KS];
   {
-    const uint16_t* qr = qbase + static_cast<int64_t>(min(qrow, p.Sq - 1)) * p.q_ss;
+    const uint16_t* qr = qbase + qhead * p.q_sh + static_cast<int64_t>(min(qrow, p.Sq - 1)) * p.q_ss;
 #pragma unroll
     for (int ks = 0; ks < S::KS; ++ks) {
       const int d0 = min(16 * ks + 8 * g, D - 8);
@@ -506,7 +567,7 @@ __global__ __launch_bounds__((64 * NW), (kMinBlocks<DP, SOFTCAP> * 4 / NW)) void
       const int key0 = kt0 + 4 * g;
       // (not in the three-workgroup head_dim 64 kernel: its 168-VGPR budget spills with
       // both paths)
-      if (kMinBlocks<DP, SOFTCAP> <= 2 && p.kmask == nullptr && kt0 + BN <= Skv) {
+      if (kMinBlocks<DP, SOFTCAP> <= 2 && kmask == nullptr && kt0 + BN <= Skv) {
         // Causal / window edges of a full tile without a block mask (the diagonal of a
         // causal sweep, the left edge of a window): element (key0 + off) is visible iff
         // lo <= off <= hi, compares against a compile-time offset per score instead of
@@ -537,7 +598,7 @@ __global__ __launch_bounds__((64 * NW), (kMinBlocks<DP, SOFTCAP> * 4 / NW)) void
         // pre-shifted by this lane half's key offset 4g, so each element tests a bit at
         // a compile-time position (no per-element 64-bit shift constants to hold)
         const uint64_t kbits =
-            p.kmask != nullptr ? kmask_row[kt0 >> 6] >> ((kt0 & 63) + 4 * g) : ~uint64_t{0};
+            kmask != nullptr ? kmask_row[kt0 >> 6] >> ((kt0 & 63) + 4 * g) : ~uint64_t{0};
 #pragma unroll
         for (int nb = 0; nb < S::NB; ++nb) {
 #pragma unroll
@@ -743,7 +804,7 @@ __global__ __launch_bounds__((64 * NW), (kMinBlocks<DP, SOFTCAP> * 4 / NW)) void
   // at or left of the wave's first row. No block mask.
   int i_lo = 0;
   int i_hi = 0;
-  if (wave_live && p.kmask == nullptr) {
+  if (wave_live && kmask == nullptr) {
     i_hi = min(nt - 2, t_full - t_begin - 2);
     if (p.causal) i_hi = min(i_hi, (qw0_abs + 1) / BN - t_begin);
     if (p.window > 0) {
@@ -770,6 +831,38 @@ __global__ __launch_bounds__((64 * NW), (kMinBlocks<DP, SOFTCAP> * 4 / NW)) void
   }
 
   const float l_tot = wave_pair_sum(l_run);
+  if constexpr (SPLIT) {
+    // partial of row (b, head, query): O normalised by this range's sum, and its lse in
+    // log2 units (-inf, and O left unwritten, when the row sees none of the range)
+    // (the row is worked out again from an opaque copy of the lane, rather than held in
+    // registers through the sweep)
+    int r = lane;
+    asm volatile("" : "+v"(r));
+    r = qw0 + (r & 31);
+    if (r < n_rows) {
+      const int hr = pack ? r / p.Sq : 0;
+      const int64_t slot =
+          ((static_cast<int64_t>(b) * p.Hq + h + hr) * p.Sq + (r - hr * p.Sq)) * sp.n_split + split;
+      if (l_tot > 0.0f) {
+        const float inv = 1.0f / l_tot;
+        float* orow = sp.ws_o + slot * D;
+#pragma unroll
+        for (int db = 0; db < SV::DB; ++db) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int d0 = 32 * db + 8 * i + 4 * g;
+            if (d0 < D) {
+              *reinterpret_cast<f32x4*>(orow + d0) =
+                  f32x4{oacc[db][4 * i + 0] * inv, oacc[db][4 * i + 1] * inv,
+                        oacc[db][4 * i + 2] * inv, oacc[db][4 * i + 3] * inv};
+            }
+          }
+        }
+      }
+      if (g == 0) sp.ws_lse[slot] = l_tot > 0.0f ? m_run * c + fast_log2(l_tot) : kNegInf;
+    }
+    return;
+  }
   if (wave_live && qrow < p.Sq) {
     float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
     float lse = l_tot > 0.0f ? (m_run * c + fast_log2(l_tot)) * kLn2 : masked_row_lse(p, qrow);
@@ -822,6 +915,57 @@ __global__ __launch_bounds__((64 * NW), (kMinBlocks<DP, SOFTCAP> * 4 / NW)) void
   }
 }
 
+// O = sum_s 2^(lse_s - max) O_s / sum_s 2^(lse_s - max) over the key ranges, in range
+// order. Each row takes D / 4 lanes of 16-byte reads (rounded up to a power of two).
+template <typename Tag>
+__global__ __launch_bounds__(256) void prefill_merge_kernel(const PrefillParams p, int log2_lanes) {
+  using E = Elem<Tag>;
+  const SplitParams& sp = p.sp;
+  const int64_t gid = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  const int64_t row = gid >> log2_lanes;
+  const int d0 = 4 * static_cast<int>(gid & ((1 << log2_lanes) - 1));
+  if (row >= static_cast<int64_t>(p.B) * p.Hq * p.Sq || d0 >= p.D) return;
+  const int64_t bh = row / p.Sq;
+  const int s = static_cast<int>(row - bh * p.Sq);
+  const int b = static_cast<int>(bh / p.Hq);
+  const int h = static_cast<int>(bh - static_cast<int64_t>(b) * p.Hq);
+  const float* lse_row = sp.ws_lse + row * sp.n_split;
+  const float* orow = sp.ws_o + row * sp.n_split * p.D + d0;
+  float mm = kNegInf;
+  for (int i = 0; i < sp.n_split; ++i) mm = fmaxf(mm, lse_row[i]);
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  float sum = 0.0f;
+  // eight ranges' partials in flight; a range the row does not see has lse -inf, weight 0,
+  // and its O (never written) is replaced by 0
+  for (int i0 = 0; i0 < sp.n_split; i0 += 8) {
+    f32x4 x[8];
+    float l[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int i = min(i0 + u, sp.n_split - 1);
+      l[u] = i0 + u < sp.n_split ? lse_row[i] : kNegInf;
+      x[u] = *reinterpret_cast<const f32x4*>(orow + static_cast<int64_t>(i) * p.D);
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const bool live = l[u] != kNegInf;
+      const float w = live ? fast_exp2(l[u] - mm) : 0.0f;
+      sum += w;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[e] = fmaf(w, live ? x[u][e] : 0.0f, acc[e]);
+    }
+  }
+  float inv = sum > 0.0f ? 1.0f / sum : 0.0f;
+  float lse = sum > 0.0f ? (mm + fast_log2(sum)) * kLn2 : masked_row_lse(p, s);
+  if (sum > 0.0f) ref_tile_floor(p, s, lse, inv);
+  uint16_t* out = p.o + b * p.o_sb + h * p.o_sh + static_cast<int64_t>(s) * p.o_ss + d0;
+  *reinterpret_cast<u32x2*>(out) =
+      u32x2{E::pack2(acc[0] * inv, acc[1] * inv), E::pack2(acc[2] * inv, acc[3] * inv)};
+  if (p.lse != nullptr && d0 == 0) {
+    p.lse[b * p.l_sb + h * p.l_sh + static_cast<int64_t>(s) * p.l_ss] = lse;
+  }
+}
+
 template <typename Tag, int DP, int DV, int BN, int NW>
 void launch_nw(const PrefillParams& p, bool softcap, int grid, hipStream_t s) {
   const size_t dyn = p.kmask != nullptr ? kLiveLdsBytes : 0;
@@ -852,6 +996,25 @@ void launch_narrow(const PrefillParams& p0, bool softcap, int grid, hipStream_t 
   const int grid8 = p.n_qt * p.B * p.Hq;
   prefill_grid_order(p.causal != 0, static_cast<int64_t>(p.B) * p.Hq, grid8, p.xcd_group, p.xcd_remap);
   launch_nw<Tag, 192, 128, kNarrowBN, 8>(p, softcap, grid8, s);
+}
+
+template <typename Tag>
+void launch_split(const PrefillParams& p, bool softcap, int grid, hipStream_t s) {
+  using Split = SplitKeys<Tag>;
+  if (p.D <= 64) {
+    launch_nw<Split, 64, 64, 64, 4>(p, softcap, grid, s);
+  } else if (p.D <= 128) {
+    launch_nw<Split, 128, 128, 64, 4>(p, softcap, grid, s);
+  } else if (p.D <= 192) {
+    launch_nw<Split, 192, 192, 32, 4>(p, softcap, grid, s);
+  } else {
+    launch_nw<Split, 256, 256, 32, 4>(p, softcap, grid, s);
+  }
+  const int64_t rows = static_cast<int64_t>(p.B) * p.Hq * p.Sq;
+  const int log2_lanes = p.D <= 64 ? 4 : (p.D <= 128 ? 5 : 6);
+  const int64_t blocks = ((rows << log2_lanes) + 255) / 256;
+  hipLaunchKernelGGL((prefill_merge_kernel<Tag>), dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, p,
+                     log2_lanes);
 }
 
 template <typename Tag>
@@ -1320,7 +1483,106 @@ void launch_f32(const PrefillParams& p, bool softcap, int grid, hipStream_t s) {
 }
 
 
+// How a call's keys are split, or n_split = 0: one workgroup sweeps all of a row's keys.
+//
+// `base` workgroups (128-row tiles over all heads) times the ranges should fill the
+// chip's slots (two workgroups per CU, one at head_dim above 192) once. Measured on
+// MI355X, bf16, us per call (device time; unsplit figures of cached calls with the
+// concatenation they need):
+//   over a cache (B, Hq/Hkv, Sq + cached, D)       unsplit   split
+//     8, 32/8, 1 + 4095, 128                          152     27.5  (4.9 TB/s of K/V)
+//     32, 32/32, 1 + 2047, 128   (base 1024)          992      202
+//     1, 32/8, 509 + 7683, 128   (base 128)           170       84
+//     1, 32/8, 1024 + 15000, 128 (base 256)           334      237
+//     4, 32/32, 512 + 512, 128   (base 512)           124       63
+//     1, 32/8, 1024 + 64, 128    (base 256)            35       41  -> not split
+//     4, 24/8, 1024 + 1000, 64   (base 768)            96       94  -> not split
+//   no cache, causal
+//     1, 4/4, 2048, 128 (base 64)                      33       24
+//     1, 2/2, 8192, 128 (base 128)                    116       64
+//     1, 8/8, 1024, 128 (base 64)                    20.4     20.3  -> not split
+//     1, 16/16, 2048, 128 (base 256)                 35.5     48.3  -> not split
+//     1, 8/8, 2048, 128, window 1024 (base 128)        25       34  -> not split
+constexpr int kSplitLeast = 256;       // shortest range over a cache (keys)
+constexpr int kSplitLeastOwn = 512;    // without one
+constexpr int kSplitMinSweep = FFA_SPLIT_MIN_KEYS;  // without a cache, shorter sweeps stay whole ...
+constexpr int kSplitMaxBase = 128;     // ... and so do launches of more workgroups
+struct SplitPlan {
+  int n_split = 0;
+  int n_qt = 0, pack = 0;
+  int lo0 = 0, lo1 = 0, len = 0, n0 = 0;
+  int64_t grid = 0;
+  size_t bytes = 0;
+};
+
+SplitPlan plan_split(const ffa_prefill_args& a) {
+  SplitPlan pl;
+  if (a.dtype == FFA_DTYPE_FP32 || a.batch == 0 || a.seqlen_q == 0 ||
+      (a.block_key_mask != nullptr && a.k_cache != nullptr) || (a.v_head_dim > 0 && a.v_head_dim < a.head_dim)) {
+    return pl;
+  }
+  const int64_t ratio = a.heads_q / a.heads_kv;
+  const int64_t sq = a.seqlen_q;
+  const int64_t cache = a.k_cache != nullptr ? a.cache_len : 0;
+  const int64_t own = a.seqlen_kv - cache;
+  const int bn = a.head_dim <= 128 ? 64 : 32;
+  const int64_t t1 = (sq + kBlockM - 1) / kBlockM;
+  const int64_t tp = (sq * ratio + kBlockM - 1) / kBlockM;
+  pl.pack = sq < kBlockM && tp < t1 * ratio;
+  pl.n_qt = static_cast<int>(pl.pack ? tp : t1);
+  const int64_t base = static_cast<int64_t>(a.batch) * a.heads_kv * (pl.pack ? tp : t1 * ratio);
+  // the keys that any row sees, in each segment
+  int64_t lo = 0, hi = a.seqlen_kv;
+  const int window = clamp_window(a.window, a.q_offset, a.seqlen_q);
+  if (window > 0) lo = a.q_offset - static_cast<int64_t>(window) + 1;
+  if (a.causal) hi = a.q_offset + sq < hi ? a.q_offset + sq : hi;
+  lo = lo < 0 ? 0 : lo;
+  if (hi <= lo) return pl;
+  const int64_t keys = hi - lo;
+  const int64_t lo1 = lo > cache ? lo - cache : 0;
+  const int64_t end0 = cache < hi ? cache : hi;
+  const int64_t end1 = hi - cache < own ? hi - cache : own;
+  int64_t n_max = (a.head_dim <= 192 ? 512 : 256) / base;
+  bool own_free = false;
+  if (cache > 0) {
+    // The partials (8 bytes written and read per row, dim and range) against the
+    // concatenation (as much per key and dim of each KV head): a full launch splits only
+    // to avoid the larger of the two, a half-empty one gains more than that.
+    n_max = n_max < 3 ? 3 : n_max;
+    if (base > kSplitMaxBase && ratio * sq * n_max > keys * (base > 512 ? 1 : 4)) return pl;
+    // a few own keys take no slot's worth of time: one more range over the cache pays
+    // unless the ranges are short already
+    own_free = end1 - lo1 <= kSplitLeast && keys > 384 * n_max * (n_max - 1);
+  } else {
+    const int64_t sweep = window > 0 && window + kBlockM < keys ? window + kBlockM : keys;
+    if (base > kSplitMaxBase || sweep < kSplitMinSweep) return pl;
+  }
+  pl.lo0 = static_cast<int>(lo / bn * bn);
+  pl.lo1 = static_cast<int>(lo1 / bn * bn);
+  const int64_t least = cache > 0 ? kSplitLeast : kSplitLeastOwn;
+  int64_t len = keys / n_max;
+  len = ((len < least ? least : len) + bn - 1) / bn * bn;
+  int64_t n1;
+  for (;;) {  // len grows by 1/16 or a tile: ends once both segments are one range each
+    pl.n0 = static_cast<int>(lo < end0 ? (end0 - pl.lo0 + len - 1) / len : 0);
+    n1 = end1 > lo1 ? (end1 - pl.lo1 + len - 1) / len : 0;
+    if (pl.n0 + (own_free ? 0 : n1) <= n_max || len >= hi) break;
+    len += (len / 16 + bn - 1) / bn * bn;
+  }
+  pl.len = static_cast<int>(len);
+  const int64_t n = pl.n0 + n1;
+  if (n < 1 || (cache == 0 && n < 2)) return pl;
+  pl.grid = base * n;
+  if (pl.grid > 0x7fffffff) return pl;
+  pl.n_split = static_cast<int>(n);
+  const int64_t rows = static_cast<int64_t>(a.batch) * a.heads_q * sq;
+  pl.bytes = static_cast<size_t>(rows) * n * (static_cast<size_t>(a.head_dim) + 1) * sizeof(float);
+  return pl;
+}
+
 }  // namespace
+
+size_t prefill_workspace_bytes(const ffa_prefill_args& a) { return plan_split(a).bytes; }
 
 int launch_prefill(const ffa_prefill_args& a, hipStream_t stream) {
   PrefillParams p{};
@@ -1392,6 +1654,39 @@ int launch_prefill(const ffa_prefill_args& a, hipStream_t stream) {
   const int64_t grid64 = static_cast<int64_t>(p.n_qt) * a.batch * a.heads_q;
   if (grid64 <= 0) return FFA_OK;
   if (grid64 > 0x7fffffff) return FFA_ERR_TOO_LARGE;
+  const SplitPlan pl = plan_split(a);
+  const bool cached = a.k_cache != nullptr && a.cache_len > 0;
+  if (pl.n_split > 0 && a.workspace != nullptr && a.workspace_bytes >= pl.bytes) {
+    SplitParams& sp = p.sp;
+    sp.kc = static_cast<const uint16_t*>(a.k_cache);
+    sp.vc = static_cast<const uint16_t*>(a.v_cache);
+    sp.kc_sb = a.k_cache_stride[0];
+    sp.kc_sh = a.k_cache_stride[1];
+    sp.kc_ss = a.k_cache_stride[2];
+    sp.vc_sb = a.v_cache_stride[0];
+    sp.vc_sh = a.v_cache_stride[1];
+    sp.vc_ss = a.v_cache_stride[2];
+    sp.cache_len = cached ? a.cache_len : 0;
+    sp.lo0 = pl.lo0;
+    sp.lo1 = pl.lo1;
+    sp.len = pl.len;
+    sp.n0 = pl.n0;
+    sp.n_split = pl.n_split;
+    sp.pack = pl.pack;
+    const int64_t rows = static_cast<int64_t>(a.batch) * a.heads_q * a.seqlen_q;
+    sp.ws_o = static_cast<float*>(a.workspace);
+    sp.ws_lse = sp.ws_o + rows * pl.n_split * a.head_dim;
+    p.n_qt = pl.n_qt;
+    p.xcd_remap = pl.grid % 8 == 0 ? 1 : 0;
+    const int grid_s = static_cast<int>(pl.grid);
+    if (a.dtype == FFA_DTYPE_BF16) {
+      launch_split<Bf16Tag>(p, softcap, grid_s, stream);
+    } else {
+      launch_split<F16Tag>(p, softcap, grid_s, stream);
+    }
+    return hipGetLastError() == hipSuccess ? FFA_OK : FFA_ERR_LAUNCH;
+  }
+  if (cached) return FFA_ERR_WORKSPACE;  // only the split kernel reads a cache in place
   const int grid = static_cast<int>(grid64);
   prefill_grid_order(p.causal != 0, static_cast<int64_t>(a.batch) * a.heads_q, grid,
                      p.xcd_group, p.xcd_remap);

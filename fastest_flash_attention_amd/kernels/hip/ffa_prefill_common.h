@@ -6,12 +6,37 @@
 #include "ffa_common.h"
 
 namespace ffa {
+
+// Marks the element tag of a kernel whose workgroups take key ranges (split launches).
+template <typename Tag>
+struct SplitKeys {};
+template <typename Tag>
+struct Elem<SplitKeys<Tag>> : Elem<Tag> {};
+template <typename Tag>
+constexpr bool kSplitKeys = false;
+template <typename Tag>
+constexpr bool kSplitKeys<SplitKeys<Tag>> = true;
+
 namespace pf {
 
 constexpr float kRescaleThresh = 8.0f;  // log2 units: the running max moves only past this
 // 16-bit kernels: the running max moves when a 16-key chunk's 8 exponentials per lane sum
 // past this (some p > 2^5), so every accumulated p stays <= 2^8.
 constexpr float kChunkLimit = 256.0f;
+
+// Key ranges of a split launch: n0 ranges of `len` keys over the cached keys from lo0 on,
+// then the rest over the call's own keys from lo1 on (positions inside each segment;
+// len, lo0 and lo1 are multiples of the key tile).
+struct SplitParams {
+  const uint16_t* kc;
+  const uint16_t* vc;
+  int64_t kc_sb, kc_sh, kc_ss;
+  int64_t vc_sb, vc_sh, vc_ss;
+  float* ws_o;    // [B][Hq][Sq][n_split][D] partial O
+  float* ws_lse;  // [B][Hq][Sq][n_split], log2 units
+  int cache_len, lo0, lo1, len, n0, n_split;
+  int pack;  // 1: the query heads of a KV head share query tiles
+};
 
 struct PrefillParams {
   const uint16_t* q;
@@ -39,6 +64,7 @@ struct PrefillParams {
   const uint64_t* kmask;  // block mask expanded to keys, [n_br][kmask_words], or null
   int kmask_words;
   const int32_t* visited;  // reference tiles visited per row block (with kmask)
+  SplitParams sp;          // split launches only
 };
 
 // Row swizzles (XOR on the 16-byte chunk index) of the K and V tiles in LDS. They make

@@ -54,6 +54,7 @@ class ResolvedForward:
     return_lse: bool
     squeezed: bool
     Dv: int = 0  # v's head dim (<= D; a narrower v is taken as zero-padded to D)
+    cache: Optional[Tuple[torch.Tensor, torch.Tensor]] = None  # K/V ahead of k, v (in place)
 
 
 @dataclass
@@ -68,7 +69,7 @@ class PrefillCall:
     lse: Optional[torch.Tensor]
     squeezed: bool
     d_user: int = 0
-    keep: tuple = ()  # device buffers the launch reads (block-mask words, counts)
+    keep: tuple = ()  # device buffers of the launch (block-mask words, KV cache, workspace)
 
 
 def _expand_block_mask(block_mask, r: "ResolvedForward", device) -> Tuple[torch.Tensor, int, torch.Tensor]:
@@ -108,15 +109,18 @@ def _expand_block_mask(block_mask, r: "ResolvedForward", device) -> Tuple[torch.
     return packed, words, visited
 
 
+def _conforms(t: torch.Tensor) -> bool:
+    return (t.stride(-1) == 1 and t.data_ptr() % 16 == 0
+            and all(st % 8 == 0 for st, n in zip(t.stride()[:3], t.shape[:3]) if n > 1))
+
+
 def _conform(t: torch.Tensor, d_pad: int) -> torch.Tensor:
     """Return ``t`` (or a copy) in the form the kernels load in 16-byte chunks: unit
     dim stride, 16-byte aligned base, batch/head/seq strides multiple of 8 elements,
     dim zero-padded to ``d_pad`` (zeros leave q.k and the stored O dims unchanged)."""
     if t.size(-1) != d_pad:
         return torch.nn.functional.pad(t, (0, d_pad - t.size(-1))).contiguous()
-    ok = (t.stride(-1) == 1 and t.data_ptr() % 16 == 0
-          and all(st % 8 == 0 for st, n in zip(t.stride()[:3], t.shape[:3]) if n > 1))
-    if ok:
+    if _conforms(t):
         return t
     out = torch.empty(t.shape, dtype=t.dtype, device=t.device)
     out.copy_(t)
@@ -136,6 +140,23 @@ def _batch_strides(t: torch.Tensor, B: int, name: str) -> list[int]:
     return st
 
 
+def _cache_fits(cache: torch.Tensor, t: torch.Tensor) -> bool:
+    """Whether the kernels can read ``cache`` where it lies, ahead of ``t``'s rows: what
+    torch.cat along dim 2 joins without a conversion, in the layout the kernels take."""
+    return (cache.dim() == 4 and t.dim() == 4 and cache.size(2) > 0
+            and cache.shape[:2] == t.shape[:2] and cache.size(3) == t.size(3)
+            and t.size(3) % 8 == 0 and cache.dtype == t.dtype and cache.device == t.device
+            and cache.stride(2) < 1 << 24 and t.stride(2) < 1 << 24 and _conforms(cache))
+
+
+def _join_cache(r: "ResolvedForward") -> None:
+    """The concatenated form of a call whose cache was kept apart."""
+    if r.cache is not None:
+        r.k = torch.cat([r.cache[0], r.k], dim=2)
+        r.v = torch.cat([r.cache[1], r.v], dim=2)
+        r.cache = None
+
+
 def resolve_forward_args(
     q: torch.Tensor,
     k: torch.Tensor,
@@ -153,8 +174,11 @@ def resolve_forward_args(
     num_kv_heads: Optional[int] = None,
     kv_cache: Optional[Tuple[torch.Tensor, torch.Tensor]] = None,
     return_lse: bool = False,
+    cache_in_place: bool = False,
 ) -> ResolvedForward:
-    """Argument resolution of the reference dispatcher (ops/attention_forward.py:65-109)."""
+    """Argument resolution of the reference dispatcher (ops/attention_forward.py:65-109).
+    With ``cache_in_place`` a ``kv_cache`` that fits k and v is kept apart (``cache``)
+    instead of being concatenated with them."""
     if config is not None:
         causal = config.causal
         softcap = config.softcap
@@ -171,15 +195,21 @@ def resolve_forward_args(
     H_kv = k.size(1)
 
     q_offset = 0
+    cache = None
+    S_kv = k.size(2)
     if kv_cache is not None:
         k_cache, v_cache = kv_cache
         if k_cache.dim() == 3:
             k_cache = k_cache.unsqueeze(1)
             v_cache = v_cache.unsqueeze(1)
-        k = torch.cat([k_cache, k], dim=2)
-        v = torch.cat([v_cache, v], dim=2)
-        q_offset = k.size(2) - S_q
-    S_kv = k.size(2)
+        S_kv += k_cache.size(2)
+        if cache_in_place and _cache_fits(k_cache, k) and _cache_fits(v_cache, v) \
+                and k_cache.size(2) == v_cache.size(2):
+            cache = (k_cache, v_cache)
+        else:
+            k = torch.cat([k_cache, k], dim=2)
+            v = torch.cat([v_cache, v], dim=2)
+        q_offset = S_kv - S_q
 
     # v may be narrower than q / k: it is then taken as zero-padded to D (the MLA
     # module's V, which the reference pads itself, modules/flash_mla.py:151-152), and
@@ -214,6 +244,7 @@ def resolve_forward_args(
         softcap=None if softcap is None else float(softcap), two_pass=bool(two_pass),
         compute_dtype=compute_dtype, block_mask=block_mask, block_q=int(bq),
         block_kv=int(bkv), return_lse=bool(return_lse), squeezed=squeezed, Dv=int(v.size(3)),
+        cache=cache,
     )
 
 
@@ -249,13 +280,22 @@ def build_prefill_args(
     a.masked_lse_mode = 1 if r.two_pass else 0
     a.dtype = dtype_code
     a.v_head_dim = r.Dv if 0 < r.Dv < r.D else 0
+    if r.cache is not None:
+        # one-row or one-head dims may have any stride; they are never stepped over
+        k_cache, v_cache = r.cache
+        a.k_cache = k_cache.data_ptr()
+        a.v_cache = v_cache.data_ptr()
+        a.cache_len = k_cache.size(2)
+        for dst, t in ((a.k_stride, r.k), (a.v_stride, r.v), (a.k_cache_stride, k_cache),
+                       (a.v_cache_stride, v_cache)):
+            dst[:] = [0 if n == 1 else st for st, n in zip(t.stride()[:3], t.shape[:3])] + [1]
     return a
 
 
 def prepare_prefill(*args, out: Optional[torch.Tensor] = None, **kwargs) -> PrefillCall:
     """Resolve arguments, check device/dtype/features, allocate outputs, build the ABI
     struct. Launches nothing."""
-    r = resolve_forward_args(*args, **kwargs)
+    r = resolve_forward_args(*args, cache_in_place=True, **kwargs)
     for name, t in (("q", r.q), ("k", r.k), ("v", r.v)):
         if t.device.type != "cuda":
             raise RuntimeError(
@@ -267,7 +307,10 @@ def prepare_prefill(*args, out: Optional[torch.Tensor] = None, **kwargs) -> Pref
     if not (r.q.dtype == r.k.dtype == r.v.dtype):
         raise TypeError(f"q/k/v dtypes differ: {r.q.dtype}, {r.k.dtype}, {r.v.dtype}")
     code = _lib.dtype_code(r.q.dtype, allow_fp32=True)
-    if r.compute_dtype is not None and r.compute_dtype != r.q.dtype:
+    rounds = r.compute_dtype is not None and r.compute_dtype != r.q.dtype
+    if rounds or r.block_mask is not None or r.Dv != r.D or code == _lib.FFA_DTYPE_FP32:
+        _join_cache(r)
+    if rounds:
         # The reference rounds q and k (not v) to compute_dtype before the fp32 product
         # (cpu_reference.py:260-262). fp32 is exact for 16-bit inputs; a 16-bit compute
         # dtype is applied as an exact round trip q -> compute_dtype -> q.dtype (every
@@ -300,15 +343,33 @@ def prepare_prefill(*args, out: Optional[torch.Tensor] = None, **kwargs) -> Pref
         if r.return_lse
         else None
     )
-    call = PrefillCall(build_prefill_args(r, out, lse, code), r.q, r.k, r.v, out, lse,
-                       r.squeezed)
-    call.d_user = d_user
+    args = build_prefill_args(r, out, lse, code)
+    keep = ()
     if r.block_mask is not None:
         packed, words, visited = _expand_block_mask(r.block_mask, r, r.q.device)
-        call.args.block_key_mask = packed.data_ptr()
-        call.args.block_key_mask_words = words
-        call.args.block_visited = visited.data_ptr()
-        call.keep = (packed, visited)
+        args.block_key_mask = packed.data_ptr()
+        args.block_key_mask_words = words
+        args.block_visited = visited.data_ptr()
+        keep = (packed, visited)
+    # Few query rows over many keys: the library splits the keys over workgroups, with a
+    # workspace, and then also reads a KV cache in place. (Without a cache it never does
+    # below FFA_SPLIT_MIN_KEYS.)
+    need = 0
+    if r.cache is not None or r.S_kv >= _lib.FFA_SPLIT_MIN_KEYS:
+        lib = _lib.load()
+        need = lib.ffa_prefill_workspace_bytes(ctypes.byref(args))
+        if r.cache is not None and need == 0:
+            _join_cache(r)
+            args = build_prefill_args(r, out, lse, code)
+            need = lib.ffa_prefill_workspace_bytes(ctypes.byref(args))
+    if need:
+        workspace = torch.empty(need, dtype=torch.uint8, device=r.q.device)
+        args.workspace = workspace.data_ptr()
+        args.workspace_bytes = need
+        keep += (workspace, r.cache)
+    call = PrefillCall(args, r.q, r.k, r.v, out, lse, r.squeezed)
+    call.d_user = d_user
+    call.keep = keep
     return call
 
 

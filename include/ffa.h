@@ -16,6 +16,7 @@
  *                              ops/attention_forward.py:112-143; the CPU branch
  *                              flash_attn_cpu_forward kernels/cpu_reference.py:132-312
  *                              defines the semantics)
+ *   ffa_prefill_workspace_bytes: sizing helper of the prefill entry point.
  *   ffa_paged_gather       <- PagedKVCache.get_kv        ops/kv_cache.py:208-232
  *   ffa_paged_decode_fwd   <- PagedKVCache.get_kv + fastest_flash_attn_forward(S_q=1)
  *                             ops/kv_cache.py:208-232, ops/attention_forward.py:23-167
@@ -48,7 +49,7 @@
 extern "C" {
 #endif
 
-#define FFA_ABI_VERSION 7
+#define FFA_ABI_VERSION 8
 
 typedef enum ffa_status {
   FFA_OK = 0,
@@ -144,9 +145,31 @@ typedef struct ffa_prefill_args {
                           MLA module builds (modules/flash_mla.py:151-152). Supported for
                           bf16 / fp16 at head_dim 129..192 with v_head_dim <= 128, a
                           multiple of 8 (FFA_ERR_UNSUPPORTED_HEAD_DIM otherwise). */
+  /* A KV cache read in place: with k_cache not NULL, keys 0 .. cache_len - 1 come from
+     k_cache / v_cache and k / v hold the other seqlen_kv - cache_len, as if they had been
+     concatenated (ops/attention_forward.py:82-89). Same dtype, heads, alignment and
+     stride rules as k / v. Only where ffa_prefill_workspace_bytes of the same call is
+     not 0, and with that workspace (FFA_ERR_WORKSPACE otherwise). */
+  const void* k_cache;
+  const void* v_cache;
+  int64_t k_cache_stride[4];
+  int64_t v_cache_stride[4];
+  int32_t cache_len;
+  /* Scratch of calls whose keys are split over workgroups; without it (NULL or too
+     small) such a call without a cache runs unsplit. 16-byte aligned. */
+  void* workspace;
+  size_t workspace_bytes;
 } ffa_prefill_args;
 
 int ffa_prefill_fwd(const ffa_prefill_args* args, void* stream);
+
+/* A call without a cache is never split below this many keys. */
+#define FFA_SPLIT_MIN_KEYS 2048
+
+/* Workspace with which ffa_prefill_fwd splits the keys of this call (few query rows over
+ * many keys: too few workgroups otherwise); 0 when it would not. Reads sizes and options
+ * only, no buffer (k_cache counts as given when it is not NULL). */
+size_t ffa_prefill_workspace_bytes(const ffa_prefill_args* args);
 
 /*
  * Paged KV pool, layout of PagedKVCache (ops/kv_cache.py:142-149):
