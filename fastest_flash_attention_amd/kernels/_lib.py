@@ -20,7 +20,7 @@ import torch  # noqa: F401  (must load torch's HIP runtime before libffa.so)
 
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libffa.so")
 
-FFA_ABI_VERSION = 8
+FFA_ABI_VERSION = 9
 FFA_DTYPE_BF16 = 0
 FFA_DTYPE_FP16 = 1
 FFA_DTYPE_FP32 = 2
@@ -65,6 +65,7 @@ class PrefillArgs(ctypes.Structure):
         ("block_key_mask_words", ctypes.c_int32),
         ("block_visited", ctypes.c_void_p),
         ("v_head_dim", ctypes.c_int32),
+        ("o_head_dim", ctypes.c_int32),
         ("k_cache", ctypes.c_void_p),
         ("v_cache", ctypes.c_void_p),
         ("k_cache_stride", _I64x4),
@@ -175,6 +176,32 @@ class MlaDecodeArgs(ctypes.Structure):
     ]
 
 
+class MlaAssembleArgs(ctypes.Structure):
+    """Mirror of ``ffa_mla_assemble_args``."""
+
+    _fields_ = [
+        ("q_nope", ctypes.c_void_p),
+        ("q_rope", ctypes.c_void_p),
+        ("kv", ctypes.c_void_p),
+        ("k_rope", ctypes.c_void_p),
+        ("cos", ctypes.c_void_p),
+        ("sin", ctypes.c_void_p),
+        ("q", ctypes.c_void_p),
+        ("k", ctypes.c_void_p),
+        ("q_nope_stride", ctypes.c_int64),
+        ("q_rope_stride", ctypes.c_int64),
+        ("kv_stride", ctypes.c_int64),
+        ("k_rope_stride", ctypes.c_int64),
+        ("batch", ctypes.c_int32),
+        ("heads", ctypes.c_int32),
+        ("seqlen", ctypes.c_int32),
+        ("head_dim", ctypes.c_int32),
+        ("rope_dim", ctypes.c_int32),
+        ("dtype", ctypes.c_int32),
+        ("table_dtype", ctypes.c_int32),
+    ]
+
+
 class AttnBwdArgs(ctypes.Structure):
     """Mirror of ``ffa_attn_bwd_args``."""
 
@@ -235,6 +262,7 @@ EXPORTS = {
         [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32],
     ),
     "ffa_mla_decode_fwd": (ctypes.c_int, [ctypes.POINTER(MlaDecodeArgs), ctypes.c_void_p]),
+    "ffa_mla_assemble": (ctypes.c_int, [ctypes.POINTER(MlaAssembleArgs), ctypes.c_void_p]),
     "ffa_attn_bwd_workspace_bytes": (
         ctypes.c_size_t, [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32],
     ),

@@ -78,6 +78,9 @@ int check_prefill_args(const ffa_prefill_args* a, bool* empty) {
   if (!valid_dtype(a->dtype) && a->dtype != FFA_DTYPE_FP32) return FFA_ERR_UNSUPPORTED_DTYPE;
   if (a->head_dim < 1 || a->head_dim > 256) return FFA_ERR_UNSUPPORTED_HEAD_DIM;
   if (const int rc = check_v_head_dim(a->v_head_dim, a->head_dim, a->dtype); rc != FFA_OK) return rc;
+  if (a->o_head_dim != 0 && a->o_head_dim != a->head_dim && a->o_head_dim != a->v_head_dim) {
+    return FFA_ERR_INVALID_ARG;
+  }
   if (a->batch < 0 || a->heads_q < 1 || a->heads_kv < 1 || a->seqlen_q < 0 || a->seqlen_kv < 0) {
     return FFA_ERR_INVALID_ARG;
   }
@@ -312,6 +315,29 @@ int ffa_mla_decode_fwd(const ffa_mla_decode_args* a, void* stream) {
   if (need > 0 && (a->workspace == nullptr || a->workspace_bytes < need)) return FFA_ERR_WORKSPACE;
   if ((reinterpret_cast<uintptr_t>(a->workspace) & 15u) != 0) return FFA_ERR_MISALIGNED;
   return ffa::launch_mla_decode(*a, static_cast<hipStream_t>(stream));
+}
+
+int ffa_mla_assemble(const ffa_mla_assemble_args* a, void* stream) {
+  if (a == nullptr) return FFA_ERR_INVALID_ARG;
+  if (!valid_dtype(a->dtype) || (a->table_dtype != a->dtype && a->table_dtype != FFA_DTYPE_FP32)) {
+    return FFA_ERR_UNSUPPORTED_DTYPE;
+  }
+  if (a->batch < 0 || a->seqlen < 0 || a->heads < 1 || a->head_dim < 1 || a->rope_dim < 1) {
+    return FFA_ERR_INVALID_ARG;
+  }
+  if (a->batch == 0 || a->seqlen == 0) return FFA_OK;
+  if (a->head_dim % 8 != 0 || a->rope_dim % 16 != 0) return FFA_ERR_MISALIGNED;
+  const void* ptrs[8] = {a->q_nope, a->q_rope, a->kv, a->k_rope, a->cos, a->sin, a->q, a->k};
+  for (const void* ptr : ptrs) {
+    if (ptr == nullptr) return FFA_ERR_INVALID_ARG;
+    if ((reinterpret_cast<uintptr_t>(ptr) & 15u) != 0) return FFA_ERR_MISALIGNED;
+  }
+  const int64_t strides[4] = {a->q_nope_stride, a->q_rope_stride, a->kv_stride, a->k_rope_stride};
+  for (const int64_t st : strides) {
+    if (st < 0) return FFA_ERR_INVALID_ARG;
+    if (st % 8 != 0) return FFA_ERR_MISALIGNED;
+  }
+  return ffa::launch_mla_assemble(*a, static_cast<hipStream_t>(stream));
 }
 
 size_t ffa_attn_bwd_workspace_bytes(int32_t batch, int32_t heads_q, int32_t seqlen_q) {

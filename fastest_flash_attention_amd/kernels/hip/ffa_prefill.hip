@@ -894,7 +894,7 @@ __global__ __launch_bounds__((64 * NW), (kMinBlocks<DP, SOFTCAP> * 4 / NW)) void
       }
       // a V narrower than head_dim is zero-padded: O's dims past it are 0 (D and Dv are
       // multiples of 8, so each 16-byte store ends at or before D)
-      for (int d0 = Dv + 8 * g; d0 < D; d0 += 16) {
+      for (int d0 = Dv + 8 * g; d0 < p.Do; d0 += 16) {
         *reinterpret_cast<u32x4*>(orow + d0) = u32x4{0u, 0u, 0u, 0u};
       }
     } else {
@@ -1613,6 +1613,7 @@ int launch_prefill(const ffa_prefill_args& a, hipStream_t stream) {
   p.Skv = a.seqlen_kv;
   p.D = a.head_dim;
   p.Dv = a.v_head_dim > 0 ? a.v_head_dim : a.head_dim;
+  p.Do = a.o_head_dim > 0 ? a.o_head_dim : a.head_dim;
   p.q_offset = a.q_offset;
   p.causal = a.causal ? 1 : 0;
   p.window = clamp_window(a.window, a.q_offset, a.seqlen_q);

@@ -65,6 +65,7 @@ struct PrefillParams {
   int kmask_words;
   const int32_t* visited;  // reference tiles visited per row block (with kmask)
   SplitParams sp;          // split launches only
+  int Do;                  // O's head dim: D, or Dv (narrow V: the zero dims are not stored)
 };
 
 // Row swizzles (XOR on the 16-byte chunk index) of the K and V tiles in LDS. They make

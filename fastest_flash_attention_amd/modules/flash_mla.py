@@ -14,9 +14,14 @@ from typing import Optional, Sequence
 import torch
 import torch.nn as nn
 
-from ..ops.attention_forward import fastest_flash_attn_forward
+from ..ops.attention_forward import forward_token_major
 from ..ops.attention_func import fastest_flash_attn_func
-from ..ops.mla_decode import MLALatentCache
+from ..ops.mla_decode import MLALatentCache, mla_assemble, mla_assembles
+
+
+def has_hooks(m: nn.Module) -> bool:
+    return bool(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
+                or m._backward_pre_hooks)
 
 
 class RotaryEmbedding(nn.Module):
@@ -42,6 +47,12 @@ class RotaryEmbedding(nn.Module):
         x1 = x[..., :half]
         x2 = x[..., half:]
         return torch.cat([x1 * cos - x2 * sin, x2 * cos + x1 * sin], dim=-1).to(x.dtype)
+
+    def tables(self, x: torch.Tensor):
+        """(cos, sin) ``[S, dim / 2]`` of ``forward(x)`` at offset 0, for x ``[B, S, *]``."""
+        pos = torch.arange(x.size(1), device=x.device, dtype=x.dtype)
+        freqs = torch.outer(pos, self.inv_freq.to(x.device))
+        return freqs.cos(), freqs.sin()
 
     def rotate_at(self, x: torch.Tensor, positions: Sequence[int]) -> torch.Tensor:
         """RoPE of one token per batch row: x ``[B, ..., D_rope]``, token of row b at
@@ -94,15 +105,23 @@ class FastestFlashMLA(nn.Module):
         the up-projection's output)."""
         B, S, _ = x.shape
         H = self.num_heads
-        q_nope = self.q_proj(x).view(B, S, H, self.head_dim).transpose(1, 2)
-        q_rope = self.rope(self.q_rope_proj(x).view(B, S, H, self.rope_dim).transpose(1, 2))
-        q = torch.cat([q_nope, q_rope], dim=-1)
-        kv = self.kv_up_proj(self.kv_down_proj(x)).view(B, S, H, 2 * self.head_dim).transpose(1, 2)
-        k_nope = kv[..., : self.head_dim]
-        v = kv[..., self.head_dim:]
-        k_rope = self.k_rope_proj(x).unsqueeze(1).expand(-1, H, -1, -1)
-        k_rope = self.rope(k_rope)
-        k = torch.cat([k_nope, k_rope], dim=-1)
+        q_nope = self.q_proj(x)
+        q_rope = self.q_rope_proj(x)
+        kv = self.kv_up_proj(self.kv_down_proj(x))
+        k_rope = self.k_rope_proj(x)
+        v = kv.view(B, S, H, 2 * self.head_dim).transpose(1, 2)[..., self.head_dim:]
+        if type(self.rope) is RotaryEmbedding and not has_hooks(self.rope) and mla_assembles(
+                q_nope, q_rope, kv, k_rope, self.head_dim, self.rope_dim):
+            # no gradient to keep: rotation and concatenation in one kernel, the same bits
+            q, k = mla_assemble(q_nope, q_rope, kv, k_rope, *self.rope.tables(x), H,
+                                self.head_dim, self.rope_dim)
+        else:
+            q_nope = q_nope.view(B, S, H, self.head_dim).transpose(1, 2)
+            q_rope = self.rope(q_rope.view(B, S, H, self.rope_dim).transpose(1, 2))
+            q = torch.cat([q_nope, q_rope], dim=-1)
+            k_nope = kv.view(B, S, H, 2 * self.head_dim).transpose(1, 2)[..., : self.head_dim]
+            k_rope = self.rope(k_rope.unsqueeze(1).expand(-1, H, -1, -1))
+            k = torch.cat([k_nope, k_rope], dim=-1)
         if not pad_v:
             return q, k, v
         v_padded = torch.nn.functional.pad(v, (0, self.rope_dim))
@@ -121,10 +140,11 @@ class FastestFlashMLA(nn.Module):
         if self.training:
             attn = fastest_flash_attn_func(q, k, v, scale=self.scale, causal=use_causal,
                                            block_size=bs or 64)
+            tokens = attn.transpose(1, 2).contiguous()
         else:
-            attn, _ = fastest_flash_attn_forward(q, k, v, scale=self.scale,
-                                                 causal=use_causal, block_size=bs)
-        return self.o_proj(attn.transpose(1, 2).contiguous().view(B, S, -1))
+            tokens, _ = forward_token_major(q, k, v, scale=self.scale, causal=use_causal,
+                                            block_size=bs)
+        return self.o_proj(tokens.view(B, S, -1))
 
     # ---- decode over the compressed latent cache (no counterpart in the reference) ----
 

@@ -280,6 +280,7 @@ def build_prefill_args(
     a.masked_lse_mode = 1 if r.two_pass else 0
     a.dtype = dtype_code
     a.v_head_dim = r.Dv if 0 < r.Dv < r.D else 0
+    a.o_head_dim = out.size(-1)
     if r.cache is not None:
         # one-row or one-head dims may have any stride; they are never stepped over
         k_cache, v_cache = r.cache
@@ -325,11 +326,7 @@ def prepare_prefill(*args, out: Optional[torch.Tensor] = None, **kwargs) -> Pref
     if r.D > 256:
         raise ValueError(f"head_dim {r.D} > 256 is not supported")
     d_pad = (r.D + 7) // 8 * 8
-    # A narrower v runs natively where the library has kernels for it (16-bit inputs,
-    # head_dim 129..192, v_head_dim <= 128 and a multiple of 8); elsewhere it is
-    # zero-padded here, which gives the same result.
-    narrow_v = (r.Dv < d_pad and code != _lib.FFA_DTYPE_FP32 and 128 < d_pad <= 192
-                and r.Dv <= 128 and r.Dv % 8 == 0)
+    narrow_v = _narrow_v(r.Dv, d_pad, r.q.dtype)
     r.q = _conform(r.q, d_pad)
     r.k = _conform(r.k, d_pad)
     r.v = _conform(r.v, r.Dv if narrow_v else d_pad)
@@ -371,6 +368,13 @@ def prepare_prefill(*args, out: Optional[torch.Tensor] = None, **kwargs) -> Pref
     call.d_user = d_user
     call.keep = keep
     return call
+
+
+def _narrow_v(Dv: int, D: int, dtype: torch.dtype) -> bool:
+    """A v narrower than q and k runs natively where the library has kernels for it (16-bit
+    inputs, head_dim 129..192, v dims <= 128 and a multiple of 8); elsewhere it is
+    zero-padded, which gives the same result."""
+    return Dv < D and dtype != torch.float32 and 128 < D <= 192 and Dv <= 128 and Dv % 8 == 0
 
 
 def launch_prefill(call: PrefillCall) -> None:
@@ -417,3 +421,21 @@ def fastest_flash_attn_forward(
         if lse is not None:
             lse = lse.squeeze(1)
     return output, lse
+
+
+def forward_token_major(
+    q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, drop_zero_dims: bool = False, **kwargs
+) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
+    """``fastest_flash_attn_forward`` of 4D inputs with the output as contiguous
+    ``[B, S, H, D]``, the order an output projection reads: the kernel writes it there, so
+    no transposed copy follows. With ``drop_zero_dims`` the output of a narrower v may come
+    with v's dims only (without the zeros past them)."""
+    B, H, S, D = q.shape
+    if D % 8 != 0:
+        out, lse = fastest_flash_attn_forward(q, k, v, **kwargs)
+        return out.transpose(1, 2).contiguous(), lse
+    width = v.size(3) if drop_zero_dims and _narrow_v(v.size(3), D, q.dtype) else D
+    tokens = torch.empty(B, S, H, width, dtype=q.dtype, device=q.device)
+    call = prepare_prefill(q, k, v, out=tokens.transpose(1, 2), **kwargs)
+    launch_prefill(call)
+    return tokens, call.lse

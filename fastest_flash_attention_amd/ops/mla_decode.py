@@ -203,6 +203,45 @@ def fastest_flash_mla_decode(
     return call.out, call.lse
 
 
+def mla_assembles(q_nope: torch.Tensor, q_rope: torch.Tensor, kv: torch.Tensor,
+                  k_rope: torch.Tensor, head_dim: int, rope_dim: int) -> bool:
+    """Whether ``mla_assemble`` takes these projections: plain 16-bit ROCm tensors of one
+    dtype in the layout it reads, with nothing to differentiate, map over or trace."""
+    if head_dim % 8 or rope_dim % 16 or torch.jit.is_tracing() or torch.compiler.is_compiling():
+        return False
+    if torch.autograd.forward_ad._current_level >= 0:
+        return False
+    dtype, device = q_nope.dtype, q_nope.device
+    if dtype not in (torch.bfloat16, torch.float16) or device.type != "cuda":
+        return False
+    return all(type(t) is torch.Tensor and not t.requires_grad and t.dtype == dtype
+               and t.device == device and not torch._C._functorch.is_functorch_wrapped_tensor(t)
+               and t.is_contiguous() and t.data_ptr() % 16 == 0
+               for t in (q_nope, q_rope, kv, k_rope))
+
+
+def mla_assemble(q_nope: torch.Tensor, q_rope: torch.Tensor, kv: torch.Tensor,
+                 k_rope: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, heads: int,
+                 head_dim: int, rope_dim: int) -> Tuple[torch.Tensor, torch.Tensor]:
+    """q and k ``[B, H, S, head_dim + rope_dim]`` of the MLA module from its projections
+    ``[B, S, *]`` (``ffa_mla_assemble``): the rope parts rotated by the tables ``[S,
+    rope_dim / 2]`` and concatenated to the others, in one kernel."""
+    B, S, _ = q_nope.shape
+    q = torch.empty(B, heads, S, head_dim + rope_dim, dtype=q_nope.dtype, device=q_nope.device)
+    k = torch.empty_like(q)
+    cos, sin = cos.contiguous(), sin.contiguous()
+    a = _lib.MlaAssembleArgs()
+    a.q_nope, a.q_rope, a.kv, a.k_rope = (t.data_ptr() for t in (q_nope, q_rope, kv, k_rope))
+    a.cos, a.sin, a.q, a.k = (t.data_ptr() for t in (cos, sin, q, k))
+    a.q_nope_stride, a.q_rope_stride = heads * head_dim, heads * rope_dim
+    a.kv_stride, a.k_rope_stride = 2 * heads * head_dim, rope_dim
+    a.batch, a.heads, a.seqlen, a.head_dim, a.rope_dim = B, heads, S, head_dim, rope_dim
+    a.dtype = _lib.dtype_code(q_nope.dtype)
+    a.table_dtype = _lib.dtype_code(cos.dtype, allow_fp32=True)
+    _lib.launch(_lib.load().ffa_mla_assemble, a, q_nope.device)
+    return q, k
+
+
 class MLALatentCache:
     """Paged cache of MLA latent rows ``[c_t | r_t]`` (latent_dim + rope_dim values per
     token, shared by all heads).

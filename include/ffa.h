@@ -29,6 +29,8 @@
  *                              no MLA decode path; this one reads the compressed latent
  *                              cache instead of up-projected K/V.
  *   ffa_mla_decode_workspace_bytes: sizing helper of the MLA decode entry point.
+ *   ffa_mla_assemble       <- q and k of FastestFlashMLA.forward (modules/flash_mla.py:
+ *                             129-152): RoPE of the rope parts and the concatenations.
  *   ffa_attn_bwd           <- fastest_flash_attn_backward   ops/attention_backward.py:19-76
  *                             (its GPU branch flash_attn_triton_backward
  *                              kernels/triton_bwd.py:122-190; the CPU branch
@@ -49,7 +51,7 @@
 extern "C" {
 #endif
 
-#define FFA_ABI_VERSION 8
+#define FFA_ABI_VERSION 9
 
 typedef enum ffa_status {
   FFA_OK = 0,
@@ -145,6 +147,9 @@ typedef struct ffa_prefill_args {
                           MLA module builds (modules/flash_mla.py:151-152). Supported for
                           bf16 / fp16 at head_dim 129..192 with v_head_dim <= 128, a
                           multiple of 8 (FFA_ERR_UNSUPPORTED_HEAD_DIM otherwise). */
+  int32_t o_head_dim;  /* 0 or head_dim: o has head_dim dims. v_head_dim (when that is
+                          narrower): o has only those, and the zero dims past them are not
+                          written (FFA_ERR_INVALID_ARG for any other value). */
   /* A KV cache read in place: with k_cache not NULL, keys 0 .. cache_len - 1 come from
      k_cache / v_cache and k / v hold the other seqlen_kv - cache_len, as if they had been
      concatenated (ops/attention_forward.py:82-89). Same dtype, heads, alignment and
@@ -357,6 +362,42 @@ typedef struct ffa_mla_decode_args {
 size_t ffa_mla_decode_workspace_bytes(int32_t batch, int32_t heads_q, int32_t dim_v,
                                       int32_t max_context_len, int32_t tokens_per_split);
 int ffa_mla_decode_fwd(const ffa_mla_decode_args* args, void* stream);
+
+/*
+ * Queries and keys of the MLA module from its projections (modules/flash_mla.py:129-152):
+ *   q[b, h, s] = [q_nope[b, s, h] | rope(q_rope[b, s, h])]
+ *   k[b, h, s] = [kv[b, s, h, 0:head_dim] | rope(k_rope[b, s])]
+ * rope(x) = [x1 cos - x2 sin | x2 cos + x1 sin] over the halves x1, x2 of x, with row s of
+ * the tables; products and sums are rounded to the tables' type, the result to dtype (the
+ * elementwise operations of the reference, bit for bit). A token's heads are contiguous:
+ * q_nope [H][head_dim], q_rope [H][rope_dim], kv [H][2 head_dim], k_rope [rope_dim]; the
+ * strides are between tokens (b S + s), in elements. q, k: contiguous [B, H, S, head_dim +
+ * rope_dim]; cos, sin: contiguous [S, rope_dim / 2]. 16-byte aligned, strides and head_dim
+ * multiples of 8, rope_dim a multiple of 16 (FFA_ERR_MISALIGNED otherwise).
+ */
+typedef struct ffa_mla_assemble_args {
+  const void* q_nope;
+  const void* q_rope;
+  const void* kv;
+  const void* k_rope;
+  const void* cos;
+  const void* sin;
+  void* q;
+  void* k;
+  int64_t q_nope_stride;
+  int64_t q_rope_stride;
+  int64_t kv_stride;
+  int64_t k_rope_stride;
+  int32_t batch;
+  int32_t heads;
+  int32_t seqlen;
+  int32_t head_dim;
+  int32_t rope_dim;
+  int32_t dtype;        /* FFA_DTYPE_BF16 or FFA_DTYPE_FP16 */
+  int32_t table_dtype;  /* of cos and sin: dtype or FFA_DTYPE_FP32 */
+} ffa_mla_assemble_args;
+
+int ffa_mla_assemble(const ffa_mla_assemble_args* args, void* stream);
 
 /*
  * Attention backward (recompute): gradients of the prefill forward above for one

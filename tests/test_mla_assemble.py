@@ -1,0 +1,105 @@
+"""The MLA module's fused query / key assembly and its token-major attention output."""
+
+from __future__ import annotations
+
+import ctypes
+
+import pytest
+import torch
+
+import fastest_flash_attention_amd as ffa
+from fastest_flash_attention_amd.kernels import _lib
+from fastest_flash_attention_amd.modules import flash_mla
+from fastest_flash_attention_amd.ops.attention_forward import forward_token_major
+from fastest_flash_attention_amd.ops.mla_decode import mla_assemble, mla_assembles
+from tests.gpu_util import require_gpu, say, seeded
+
+BF16, F16 = torch.bfloat16, torch.float16
+
+
+def test_abi_checks():
+    lib = _lib.load()
+
+    def rc(**kw):
+        a = _lib.MlaAssembleArgs()
+        base = dict(batch=1, heads=2, seqlen=3, head_dim=64, rope_dim=16, dtype=0, table_dtype=2,
+                    q_nope_stride=128, q_rope_stride=32, kv_stride=256, k_rope_stride=16)
+        for name in ("q_nope", "q_rope", "kv", "k_rope", "cos", "sin", "q", "k"):
+            base[name] = 16
+        for name, val in {**base, **kw}.items():
+            setattr(a, name, val)
+        return lib.ffa_mla_assemble(ctypes.byref(a), None)
+
+    assert lib.ffa_mla_assemble(None, None) == -1
+    assert rc(dtype=2) == -2 and rc(table_dtype=1) == -2
+    assert rc(batch=-1) == -1 and rc(heads=0) == -1 and rc(cos=None) == -1 and rc(kv_stride=-8) == -1
+    assert rc(head_dim=60) == -4 and rc(rope_dim=24) == -4 and rc(q=24) == -4 and rc(kv_stride=12) == -4
+    assert rc(batch=0, q=None) == 0 and rc(seqlen=0) == 0
+
+
+def test_cpu_and_differentiable_inputs_take_the_general_path():
+    t = torch.zeros(1, 2, 64, dtype=BF16)
+    assert not mla_assembles(t, t, t, t, 64, 16)          # not on a ROCm device
+    m = ffa.FastestFlashMLA(64, 2, head_dim=16, latent_dim=32, rope_dim=16).to(BF16).eval()
+    q, k, v = m.project_qkv(torch.randn(1, 5, 64).to(BF16))
+    assert q.requires_grad and k.requires_grad and v.requires_grad
+
+
+def general(m, x):
+    """project_qkv with the elementwise operations (the path of differentiable inputs)."""
+    with torch.enable_grad():
+        return [t.detach() for t in m.project_qkv(x, pad_v=False)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", [BF16, F16])
+@pytest.mark.parametrize("rope32", [False, True])
+@pytest.mark.parametrize("B,S,H,hd,R", [(1, 1, 1, 128, 64), (2, 77, 3, 128, 64), (1, 300, 2, 8, 16),
+                                        (3, 33, 5, 72, 48), (1, 5000, 1, 64, 32)])
+def test_same_bits_as_the_elementwise_operations(dt, rope32, B, S, H, hd, R):
+    require_gpu()
+    say(f"mla assemble B{B} S{S} H{H} hd{hd} R{R} {dt} rope32={rope32}")
+    torch.manual_seed(0)
+    m = ffa.FastestFlashMLA(96, H, head_dim=hd, latent_dim=64, rope_dim=R).cuda().to(dt).eval()
+    if rope32:
+        m.rope = flash_mla.RotaryEmbedding(R).cuda()
+    x = seeded((B, S, 96), dt, 5).cuda()
+    want = general(m, x)
+    with torch.no_grad():
+        raw = (m.q_proj(x), m.q_rope_proj(x), m.kv_up_proj(m.kv_down_proj(x)), m.k_rope_proj(x))
+        assert mla_assembles(*raw, hd, R)
+        got = m.project_qkv(x, pad_v=False)
+    for g, w in zip(got, want):
+        assert g.shape == w.shape and torch.equal(g, w)
+
+
+@pytest.mark.gpu
+def test_infinities_and_signed_zeros_pass_through():
+    require_gpu()
+    dt, B, S, H, hd, R = F16, 1, 4, 2, 8, 16
+    raw = [seeded((B, S, n), dt, i).cuda() for i, n in enumerate((H * hd, H * R, H * 2 * hd, R))]
+    for t in raw:
+        t.view(-1)[0], t.view(-1)[1], t.view(-1)[2] = float("inf"), float("nan"), -0.0
+    rope = flash_mla.RotaryEmbedding(R).cuda()
+    q, k = mla_assemble(*raw, *rope.tables(raw[0]), H, hd, R)
+    qw = torch.cat([raw[0].view(B, S, H, hd).transpose(1, 2),
+                    rope(raw[1].view(B, S, H, R).transpose(1, 2))], dim=-1)
+    kw = torch.cat([raw[2].view(B, S, H, 2 * hd).transpose(1, 2)[..., :hd],
+                    rope(raw[3].unsqueeze(1).expand(-1, H, -1, -1))], dim=-1)
+    assert torch.equal(q.nan_to_num(7.0), qw.nan_to_num(7.0))
+    assert torch.equal(k.nan_to_num(7.0), kw.nan_to_num(7.0))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("S", [1, 130, 4097])
+@pytest.mark.parametrize("D,Dv,H", [(192, 128, 3), (136, 8, 2), (192, 192, 2), (64, 64, 2), (20, 20, 2)])
+def test_token_major_output(S, D, Dv, H):
+    require_gpu()
+    say(f"token major S{S} D{D} Dv{Dv}")
+    q, k, v = (seeded((1, H, S, d), BF16, i).cuda() for i, d in enumerate((D, D, Dv)))
+    want, lw = ffa.fastest_flash_attn_forward(q, k, v, causal=True, return_lse=True)
+    want = want.transpose(1, 2)
+    got, lg = forward_token_major(q, k, v, causal=True, return_lse=True)
+    assert got.is_contiguous() and torch.equal(got, want) and torch.equal(lg, lw)
+    got, _ = forward_token_major(q, k, v, causal=True, drop_zero_dims=True)
+    assert torch.equal(got, want[..., :got.size(-1)]) and not want[..., got.size(-1):].any()
