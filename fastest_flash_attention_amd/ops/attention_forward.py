@@ -326,13 +326,13 @@ def prepare_prefill(*args, out: Optional[torch.Tensor] = None, **kwargs) -> Pref
     if r.D > 256:
         raise ValueError(f"head_dim {r.D} > 256 is not supported")
     d_pad = (r.D + 7) // 8 * 8
-    narrow_v = _narrow_v(r.Dv, d_pad, r.q.dtype)
+    narrow = narrow_v(r.Dv, d_pad, r.q.dtype)
     r.q = _conform(r.q, d_pad)
     r.k = _conform(r.k, d_pad)
-    r.v = _conform(r.v, r.Dv if narrow_v else d_pad)
+    r.v = _conform(r.v, r.Dv if narrow else d_pad)
     d_user = r.D
     r.D = d_pad
-    r.Dv = r.Dv if narrow_v else d_pad
+    r.Dv = r.Dv if narrow else d_pad
     if out is None or d_pad != d_user:
         out = torch.empty((r.B, r.H_q, r.S_q, d_pad), dtype=r.q.dtype, device=r.q.device)
     lse = (
@@ -370,7 +370,7 @@ def prepare_prefill(*args, out: Optional[torch.Tensor] = None, **kwargs) -> Pref
     return call
 
 
-def _narrow_v(Dv: int, D: int, dtype: torch.dtype) -> bool:
+def narrow_v(Dv: int, D: int, dtype: torch.dtype) -> bool:
     """A v narrower than q and k runs natively where the library has kernels for it (16-bit
     inputs, head_dim 129..192, v dims <= 128 and a multiple of 8); elsewhere it is
     zero-padded, which gives the same result."""
@@ -434,7 +434,7 @@ def forward_token_major(
     if D % 8 != 0:
         out, lse = fastest_flash_attn_forward(q, k, v, **kwargs)
         return out.transpose(1, 2).contiguous(), lse
-    width = v.size(3) if drop_zero_dims and _narrow_v(v.size(3), D, q.dtype) else D
+    width = v.size(3) if drop_zero_dims and narrow_v(v.size(3), D, q.dtype) else D
     tokens = torch.empty(B, S, H, width, dtype=q.dtype, device=q.device)
     call = prepare_prefill(q, k, v, out=tokens.transpose(1, 2), **kwargs)
     launch_prefill(call)

@@ -103,3 +103,25 @@ def test_token_major_output(S, D, Dv, H):
     assert got.is_contiguous() and torch.equal(got, want) and torch.equal(lg, lw)
     got, _ = forward_token_major(q, k, v, causal=True, drop_zero_dims=True)
     assert torch.equal(got, want[..., :got.size(-1)]) and not want[..., got.size(-1):].any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,S", [(1, 4095), (1, 4096), (2, 2100)])
+def test_o_proj_without_the_zero_columns(B, S):
+    """From 4096 rows on the output projection skips the columns that meet V's padding: the
+    same sums (in another order) as the whole product; a hooked projection is called as it
+    is."""
+    require_gpu()
+    say(f"o_proj B{B} S{S}")
+    torch.manual_seed(1)
+    m = ffa.FastestFlashMLA(128, 2, head_dim=128, latent_dim=64, rope_dim=64).cuda().to(BF16).eval()
+    x = seeded((B, S, 128), BF16, 3).cuda()
+    calls = []
+    with torch.no_grad():
+        got = m(x)
+        hook = m.o_proj.register_forward_pre_hook(lambda mod, args: calls.append(args[0].shape))
+        whole = m(x)
+        hook.remove()
+    assert calls == [(B, S, 2 * 192)]
+    # bf16 outputs of one fp32 sum: at most a rounding of the last bit apart
+    assert (got - whole).abs().max() <= 2 ** -7 * whole.abs().max()
