@@ -20,7 +20,7 @@ import torch  # noqa: F401  (must load torch's HIP runtime before libffa.so)
 
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libffa.so")
 
-FFA_ABI_VERSION = 9
+FFA_ABI_VERSION = 10
 FFA_DTYPE_BF16 = 0
 FFA_DTYPE_FP16 = 1
 FFA_DTYPE_FP32 = 2
@@ -73,6 +73,25 @@ class PrefillArgs(ctypes.Structure):
         ("cache_len", ctypes.c_int32),
         ("workspace", ctypes.c_void_p),
         ("workspace_bytes", ctypes.c_size_t),
+    ]
+
+
+class BlockMaskArgs(ctypes.Structure):
+    """Mirror of ``ffa_block_mask_args``."""
+
+    _fields_ = [
+        ("mask", ctypes.c_void_p),
+        ("key_mask", ctypes.c_void_p),
+        ("visited", ctypes.c_void_p),
+        ("mask_stride", ctypes.c_int64),
+        ("words", ctypes.c_int32),
+        ("seqlen_q", ctypes.c_int32),
+        ("seqlen_kv", ctypes.c_int32),
+        ("block_q", ctypes.c_int32),
+        ("block_kv", ctypes.c_int32),
+        ("q_offset", ctypes.c_int32),
+        ("causal", ctypes.c_int32),
+        ("window", ctypes.c_int32),
     ]
 
 
@@ -246,6 +265,7 @@ class AttnBwdArgs(ctypes.Structure):
 EXPORTS = {
     "ffa_prefill_fwd": (ctypes.c_int, [ctypes.POINTER(PrefillArgs), ctypes.c_void_p]),
     "ffa_prefill_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(PrefillArgs)]),
+    "ffa_block_mask_expand": (ctypes.c_int, [ctypes.POINTER(BlockMaskArgs), ctypes.c_void_p]),
     "ffa_paged_gather": (ctypes.c_int, [ctypes.POINTER(PagedGatherArgs), ctypes.c_void_p]),
     "ffa_paged_append": (ctypes.c_int, [ctypes.POINTER(PagedAppendArgs), ctypes.c_void_p]),
     "ffa_paged_decode_num_splits": (ctypes.c_int32, [ctypes.c_int32, ctypes.c_int32]),

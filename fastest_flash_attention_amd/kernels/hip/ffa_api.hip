@@ -209,6 +209,26 @@ size_t ffa_prefill_workspace_bytes(const ffa_prefill_args* a) {
   return ffa::prefill_workspace_bytes(*a);
 }
 
+int ffa_block_mask_expand(const ffa_block_mask_args* a, void* stream) {
+  if (a == nullptr) return FFA_ERR_INVALID_ARG;
+  if (a->seqlen_q < 0 || a->seqlen_kv < 0 || a->block_q < 1 || a->block_kv < 1 || a->mask_stride < 0 ||
+      static_cast<int64_t>(a->words) * 64 < a->seqlen_kv || a->words < 1) {
+    return FFA_ERR_INVALID_ARG;
+  }
+  if (a->seqlen_q == 0) return FFA_OK;
+  if (a->key_mask == nullptr || a->visited == nullptr || (a->seqlen_kv > 0 && a->mask == nullptr)) {
+    return FFA_ERR_INVALID_ARG;
+  }
+  if ((reinterpret_cast<uintptr_t>(a->key_mask) & 7u) != 0) return FFA_ERR_MISALIGNED;
+  // tile bounds are 32-bit products in the kernel
+  const int64_t limit = ffa::kMaxPos;
+  if (a->seqlen_q > limit || a->seqlen_kv > limit || a->block_q > limit || a->block_kv > limit ||
+      a->words > limit / 64 + 1) {
+    return FFA_ERR_TOO_LARGE;
+  }
+  return ffa::launch_block_mask_expand(*a, static_cast<hipStream_t>(stream));
+}
+
 int ffa_paged_gather(const ffa_paged_gather_args* a, void* stream) {
   if (a == nullptr) return FFA_ERR_INVALID_ARG;
   if (a->elem_bytes != 2 && a->elem_bytes != 4) return FFA_ERR_UNSUPPORTED_DTYPE;

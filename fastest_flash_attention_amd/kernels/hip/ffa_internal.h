@@ -13,6 +13,9 @@ namespace ffa {
 size_t prefill_workspace_bytes(const ffa_prefill_args& a);
 int launch_prefill(const ffa_prefill_args& a, hipStream_t stream);
 
+// Block mask -> key bits and visited counts.
+int launch_block_mask_expand(const ffa_block_mask_args& a, hipStream_t stream);
+
 // Paged decode: split kernel + logsumexp combine kernel.
 int32_t decode_num_splits(int32_t max_context_len, int32_t tokens_per_split);
 int32_t decode_tokens_per_split(int32_t tokens_per_split);

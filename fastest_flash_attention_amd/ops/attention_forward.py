@@ -78,7 +78,7 @@ def _expand_block_mask(block_mask, r: "ResolvedForward", device) -> Tuple[torch.
     block_kv] (keys >= S_kv clear), plus the number of tiles the reference loop visits
     per query tile (mask set, not past the causal bound, not left of the window;
     cpu_reference.py:215-231), which fixes the LSE sentinel of rows with no visible
-    key. All on the device."""
+    key. One launch on a ROCm device; the elementwise form states what it computes."""
     bq, bkv = r.block_q, r.block_kv
     n_br = math.ceil(r.S_q / bq)
     n_bc = math.ceil(r.S_kv / bkv) if r.S_kv > 0 else 0
@@ -86,8 +86,11 @@ def _expand_block_mask(block_mask, r: "ResolvedForward", device) -> Tuple[torch.
     if bm.dim() != 2 or bm.shape[0] < n_br or bm.shape[1] < n_bc:
         raise ValueError(f"block_mask of shape {tuple(bm.shape)} does not cover the "
                          f"[{n_br}, {n_bc}] tiles of block size ({bq}, {bkv})")
-    bm = bm[:n_br, :n_bc].to(device=device, dtype=torch.bool)
+    bm = bm[:n_br, :n_bc].to(dtype=torch.bool)
     words = max(1, math.ceil(r.S_kv / 64))
+    if device.type == "cuda":
+        return _expand_block_mask_device(bm, r, device, n_br, words)
+    bm = bm.to(device)
     keys = torch.arange(words * 64, device=device)
     if n_bc > 0:
         bits = bm[:, torch.clamp(keys // bkv, max=n_bc - 1)] & (keys < r.S_kv)[None, :]
@@ -106,6 +109,28 @@ def _expand_block_mask(block_mask, r: "ResolvedForward", device) -> Tuple[torch.
         k_last = torch.clamp((j + 1) * bkv, max=r.S_kv) - 1
         visit &= k_last[None, :] >= (q_first - r.sliding_window + 1)[:, None]
     visited = visit.sum(dim=1).to(torch.int32).contiguous()
+    return packed, words, visited
+
+
+def _expand_block_mask_device(bm, r: "ResolvedForward", device, n_br: int, words: int):
+    """``_expand_block_mask`` in one launch of ``ffa_block_mask_expand``. A host mask goes
+    over through pinned memory, so the call does not wait for the work queued before it."""
+    if bm.device.type == "cpu" and bm.numel() and not torch.cuda.is_current_stream_capturing():
+        bm = bm.contiguous().pin_memory().to(device, non_blocking=True)
+    else:
+        bm = bm.to(device).contiguous()
+    packed = torch.empty(n_br, words, dtype=torch.int64, device=device)
+    visited = torch.empty(n_br, dtype=torch.int32, device=device)
+    a = _lib.BlockMaskArgs()
+    a.mask, a.key_mask, a.visited = bm.data_ptr(), packed.data_ptr(), visited.data_ptr()
+    a.mask_stride = bm.size(1)
+    a.words = words
+    a.seqlen_q, a.seqlen_kv = r.S_q, r.S_kv
+    # (a tile or a window beyond the sequence is one that ends with it)
+    a.block_q, a.block_kv = min(r.block_q, max(r.S_q, 1)), min(r.block_kv, max(r.S_kv, 1))
+    a.q_offset, a.causal = r.q_offset, 1 if r.causal else 0
+    a.window = min(r.sliding_window, 2 ** 31 - 1) if r.sliding_window is not None else 0
+    _lib.launch(_lib.load().ffa_block_mask_expand, a, device)
     return packed, words, visited
 
 

@@ -17,6 +17,9 @@
  *                              flash_attn_cpu_forward kernels/cpu_reference.py:132-312
  *                              defines the semantics)
  *   ffa_prefill_workspace_bytes: sizing helper of the prefill entry point.
+ *   ffa_block_mask_expand  <- the block_mask tests of the reference loop
+ *                             (kernels/cpu_reference.py:215-231), as the buffers
+ *                             ffa_prefill_fwd reads.
  *   ffa_paged_gather       <- PagedKVCache.get_kv        ops/kv_cache.py:208-232
  *   ffa_paged_decode_fwd   <- PagedKVCache.get_kv + fastest_flash_attn_forward(S_q=1)
  *                             ops/kv_cache.py:208-232, ops/attention_forward.py:23-167
@@ -51,7 +54,7 @@
 extern "C" {
 #endif
 
-#define FFA_ABI_VERSION 9
+#define FFA_ABI_VERSION 10
 
 typedef enum ffa_status {
   FFA_OK = 0,
@@ -175,6 +178,29 @@ int ffa_prefill_fwd(const ffa_prefill_args* args, void* stream);
  * many keys: too few workgroups otherwise); 0 when it would not. Reads sizes and options
  * only, no buffer (k_cache counts as given when it is not NULL). */
 size_t ffa_prefill_workspace_bytes(const ffa_prefill_args* args);
+
+/*
+ * block_key_mask and block_visited of ffa_prefill_args from a tile mask: mask[i *
+ * mask_stride + j] != 0 keeps key tile j (block_kv keys) for query tile i (block_q rows).
+ * words >= ceil(seqlen_kv / 64); bits of keys >= seqlen_kv are clear. seqlen_q, q_offset,
+ * causal and window are the call's.
+ */
+typedef struct ffa_block_mask_args {
+  const uint8_t* mask;   /* [ceil(seqlen_q / block_q)][>= ceil(seqlen_kv / block_kv)] */
+  uint64_t* key_mask;    /* [ceil(seqlen_q / block_q)][words] */
+  int32_t* visited;      /* [ceil(seqlen_q / block_q)] */
+  int64_t mask_stride;
+  int32_t words;
+  int32_t seqlen_q;
+  int32_t seqlen_kv;
+  int32_t block_q;
+  int32_t block_kv;
+  int32_t q_offset;
+  int32_t causal;
+  int32_t window;        /* <= 0: none */
+} ffa_block_mask_args;
+
+int ffa_block_mask_expand(const ffa_block_mask_args* args, void* stream);
 
 /*
  * Paged KV pool, layout of PagedKVCache (ops/kv_cache.py:142-149):
