@@ -298,3 +298,41 @@ def test_split_calls_under_capture_and_on_two_streams():
     for per in outs:
         for oo, ll in per:
             assert torch.equal(oo, o) and torch.equal(ll, lse)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["band", "runs", "causal"])
+@pytest.mark.parametrize("D,softcap", [(128, None), (64, 20.0)])
+def test_block_mask_runs(name, D, softcap):
+    """Runs of whole, consecutive tiles in the live-tile list take the fast steps: runs that
+    start at odd positions, end inside and cross the 64 positions looked at together."""
+    require_gpu()
+    S, Hq, n = 4400, 4, 69  # 140 workgroups: not split
+    bm = torch.zeros(n, n, dtype=torch.bool)
+    i, j = torch.arange(n)[:, None], torch.arange(n)[None, :]
+    if name == "band":
+        bm |= (j == 0) | ((i - j).abs() <= 9)
+    elif name == "runs":  # 3, then 5, then the rest with holes
+        bm |= (j < 3) | ((j >= 5) & (j < 10)) | ((j > 11) & (j % 13 != 0))
+    else:
+        bm |= j <= i
+        bm[:, 66] = False
+    say(f"mask runs {name} D{D} cap{softcap}")
+    q = seeded((1, Hq, S, D), BF16, 1)
+    k, v = (seeded((1, 1, S, D), BF16, s) for s in (2, 3))
+    kw = dict(causal=name != "runs", num_kv_heads=1, softcap=softcap, block_size=64)
+    args = (q.cuda(), k.cuda(), v.cuda())
+    assert not af.prepare_prefill(*args, block_mask=bm, **kw).args.workspace
+    o, lse = ffa.fastest_flash_attn_forward(*args, block_mask=bm, return_lse=True, **kw)
+    rows = np.r_[0:70, 1000:1040, 2170:2240, 4300:4400]  # in whole 64-row tiles of the mask
+    tiles = sorted({r // 64 for r in rows})
+    for t in tiles:  # one query tile of the mask at a time, at its offset
+        a, b = t * 64, min(t * 64 + 64, S)
+        off = a
+        sub = bm[t:t + 1].numpy()
+        ro, rl = rf.flash_attn_cpu_forward(
+            np32(q[:, :, a:b]), np.repeat(np32(k), Hq, 1), np.repeat(np32(v), Hq, 1),
+            scale=1 / math.sqrt(D), causal=kw["causal"], block_q=64, block_kv=64, block_mask=sub,
+            softcap=softcap, sliding_window=None, two_pass=False, compute_dtype=None, q_offset=off,
+            return_lse=True)
+        assert_parity(o[:, :, a:b], ro, lse[:, :, a:b], rl, f"{name} tile {t}")
