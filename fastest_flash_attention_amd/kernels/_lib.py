@@ -20,7 +20,7 @@ import torch  # noqa: F401  (must load torch's HIP runtime before libffa.so)
 
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libffa.so")
 
-FFA_ABI_VERSION = 10
+FFA_ABI_VERSION = 11
 FFA_DTYPE_BF16 = 0
 FFA_DTYPE_FP16 = 1
 FFA_DTYPE_FP32 = 2
@@ -286,6 +286,7 @@ EXPORTS = {
     "ffa_attn_bwd_workspace_bytes": (
         ctypes.c_size_t, [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32],
     ),
+    "ffa_attn_bwd_split_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(AttnBwdArgs)]),
     "ffa_attn_bwd": (ctypes.c_int, [ctypes.POINTER(AttnBwdArgs), ctypes.c_void_p]),
     "ffa_strerror": (ctypes.c_char_p, [ctypes.c_int]),
     "ffa_abi_version": (ctypes.c_int, []),

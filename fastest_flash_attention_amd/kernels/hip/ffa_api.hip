@@ -365,6 +365,17 @@ size_t ffa_attn_bwd_workspace_bytes(int32_t batch, int32_t heads_q, int32_t seql
   return ffa::attn_bwd_workspace_bytes(batch, heads_q, seqlen_q);
 }
 
+size_t ffa_attn_bwd_split_workspace_bytes(const ffa_attn_bwd_args* a) {
+  if (a == nullptr || a->batch < 0 || a->heads_q < 1 || a->heads_kv < 1 ||
+      a->heads_q % a->heads_kv != 0 || a->seqlen_q < 0 || a->seqlen_kv < 0 || a->head_dim < 1 ||
+      a->head_dim > 256 || a->v_head_dim < 0 || a->v_head_dim > a->head_dim ||
+      a->seqlen_q > ffa::kMaxPos || a->seqlen_kv > ffa::kMaxPos || a->q_offset > ffa::kMaxPos ||
+      a->q_offset < -ffa::kMaxPos) {
+    return 0;
+  }
+  return ffa::attn_bwd_split_workspace_bytes(*a);
+}
+
 int ffa_attn_bwd(const ffa_attn_bwd_args* a, void* stream) {
   if (a == nullptr) return FFA_ERR_INVALID_ARG;
   if (!valid_dtype(a->dtype) && a->dtype != FFA_DTYPE_FP32) return FFA_ERR_UNSUPPORTED_DTYPE;

@@ -10,8 +10,8 @@
 // head sum over the q heads of its group. A row whose LSE is -inf (no visible key in
 // the two-pass forward) contributes nothing (P = 0).
 //
-// Three launches on the caller's stream, no atomics (results are run-to-run
-// deterministic):
+// Three launches on the caller's stream (four where dK/dV sweeps are cut into parts), no
+// atomics (results are run-to-run deterministic):
 //   1. bwd_pre_kernel   lse2 = lse * log2e (+inf for -inf rows and the padding rows up
 //                       to the next 128-row boundary) and D_i, both fp32, into the
 //                       workspace [B * Hq][Sq_pad].
@@ -86,7 +86,27 @@ struct BwdParams {
   int xcd_remap_dq, xcd_remap_dkv;
   int xcd_group_dq, xcd_group_dkv;  // > 0: units per interleaved group on one XCD
   int Dv;  // V's (and dV's) head dim, <= D: V is taken as zero-padded to D
+  // dK/dV sweeps cut into parts of part_len tiles, at most n_part of them (1: none is cut)
+  int n_part, part_len;
+  float* part;  // [B * Hkv][n_kt][n_part][128 keys][D + Dv] fp32 dK | dV of cut sweeps
 };
+
+constexpr int kCutMaxDim = 192;  // head_dim up to which dK/dV sweeps can be cut
+
+// The 32-row q tiles [first, first + n) whose rows may see key tile kt (128 keys): causal
+// q_abs >= key, window q_abs <= key + window - 1.
+__host__ __device__ inline void dkv_rows(const BwdParams& p, int kt, int& first, int& n) {
+  const int k0 = kt * kDkvKeys;
+  const int k_last = (k0 + kDkvKeys < p.Skv ? k0 + kDkvKeys : p.Skv) - 1;
+  const int q_lo = p.causal && k0 > p.q_offset ? k0 - p.q_offset : 0;
+  int q_hi = p.Sq;
+  if (p.window > 0) {
+    const int64_t hi = static_cast<int64_t>(k_last) + p.window - p.q_offset;
+    q_hi = hi < q_hi ? static_cast<int>(hi) : q_hi;
+  }
+  first = q_lo / kDkvRows;
+  n = q_hi > q_lo ? (q_hi + kDkvRows - 1) / kDkvRows - first : 0;
+}
 
 // Workgroup -> (unit u = batch x head, tile j; j = 0 the heaviest causal tile): the
 // XCD-aware order of ffa_grid.h, the same as the forward kernel's grid, with the
@@ -297,7 +317,14 @@ constexpr int kBwdMinBlocks = DP <= 128 ? 2 : 1;
 // over a V of at most 128 dims (the MLA module's V, which the reference zero-pads):
 // with V's padding zero, dP = dO V^T needs dO's first DV dims only, and dV's padding
 // dims are not outputs, so dP and dV run over DV dims.
-template <typename Tag, int DP, int DV, bool SOFTCAP>
+//
+// CUT: a workgroup's sweep is the group's q heads times its q tiles, so few KV heads give
+// few workgroups, and causal ones of very uneven length: the launch then lasts as long as
+// the heaviest. With CUT, sweeps longer than part_len tiles are cut into parts of that
+// length, one workgroup each, whose fp32 sums bwd_dkdv_sum_kernel adds (plan_dkv_parts has
+// the rule and what it measured). A variant of its own: the part's bounds cost the uncut
+// kernel 2-4 % (8 % at head_dim 64), and at head_dim 256 they spill.
+template <typename Tag, int DP, int DV, bool SOFTCAP, bool CUT>
 __global__ __launch_bounds__(kThreads, kBwdMinBlocks<DP>) void bwd_dkdv_kernel(const BwdParams p) {
   using S = BShape<DP>;   // Q, K, dK
   using SV = BShape<DV>;  // dO, V, dV
@@ -320,7 +347,12 @@ __global__ __launch_bounds__(kThreads, kBwdMinBlocks<DP>) void bwd_dkdv_kernel(c
   const int g = lane >> 5;
 
   int bh, kt;  // causal: low key tiles are seen by the most rows (heaviest first)
-  bwd_item(blockIdx.x, p.n_kt, p.xcd_group_dkv, p.xcd_remap_dkv, bh, kt);
+  int part = 0;
+  bwd_item(blockIdx.x, CUT ? p.n_kt * p.n_part : p.n_kt, p.xcd_group_dkv, p.xcd_remap_dkv, bh, kt);
+  if constexpr (CUT) {
+    part = kt % p.n_part;
+    kt /= p.n_part;
+  }
   const int b = bh / p.Hkv;
   const int hk = bh - b * p.Hkv;
   const int D = p.D;
@@ -330,18 +362,15 @@ __global__ __launch_bounds__(kThreads, kBwdMinBlocks<DP>) void bwd_dkdv_kernel(c
   const int kw0 = k0 + wave * 32;
   const int key = kw0 + l32;
   const bool wave_live = kw0 < p.Skv;
-  const int k_last = min(k0 + kDkvKeys, p.Skv) - 1;
 
-  // q rows whose visible keys meet [k0, k_last]: causal q_abs >= key, window
-  // q_abs <= key + window - 1.
-  const int q_lo = p.causal ? max(0, k0 - p.q_offset) : 0;
-  const int q_hi = p.window > 0
-                       ? static_cast<int>(min<int64_t>(Sq, static_cast<int64_t>(k_last) + p.window -
-                                                               p.q_offset))
-                       : Sq;
-  const int qt_begin = q_lo / kDkvRows;
-  const int ntq = q_hi > q_lo ? (q_hi + kDkvRows - 1) / kDkvRows - qt_begin : 0;
+  int qt_begin, ntq;
+  dkv_rows(p, kt, qt_begin, ntq);
   const int nit = ntq * p.ratio;
+  // this workgroup's part of the sweep (every part but the first may be empty)
+  const bool cut = CUT && nit > p.part_len;
+  const int it_begin = CUT ? part * p.part_len : 0;
+  const int it_end = CUT ? min(nit, it_begin + p.part_len) : nit;
+  if (CUT && part > 0 && it_begin >= nit) return;
 
   const float c = SOFTCAP ? p.cap_mul : p.score_mul;
 
@@ -403,8 +432,8 @@ __global__ __launch_bounds__(kThreads, kBwdMinBlocks<DP>) void bwd_dkdv_kernel(c
   // Tiles are visited q head by q head of the group, q tiles ascending within each.
   // The next tile to issue is tracked incrementally (head r of the group, tile index
   // qi, running byte pointers) instead of dividing the iteration index.
-  int is_r = 0;
-  int is_qi = 0;
+  int is_r = it_begin > 0 ? it_begin / ntq : 0;
+  int is_qi = it_begin - is_r * ntq;
   const char* is_qb = nullptr;
   const char* is_db = nullptr;
   int64_t is_ws = 0;
@@ -412,7 +441,7 @@ __global__ __launch_bounds__(kThreads, kBwdMinBlocks<DP>) void bwd_dkdv_kernel(c
   const int64_t do_tile_bytes = static_cast<int64_t>(kDkvRows) * p.do_ss * 2;
   auto is_head = [&]() {
     const int hq = hk * p.ratio + is_r;
-    const int q0 = qt_begin * kDkvRows;
+    const int q0 = (CUT ? qt_begin + is_qi : qt_begin) * kDkvRows;
     is_qb = reinterpret_cast<const char*>(p.q + b * p.q_sb + hq * p.q_sh +
                                           static_cast<int64_t>(q0) * p.q_ss);
     is_db = reinterpret_cast<const char*>(p.dout + b * p.do_sb + hq * p.do_sh +
@@ -490,13 +519,13 @@ __global__ __launch_bounds__(kThreads, kBwdMinBlocks<DP>) void bwd_dkdv_kernel(c
     }
   }
 
-  if (nit > 0) issue(0);
-  int cur_qi = 0;  // q tile index (within [0, ntq)) of iteration it
-  for (int it = 0; it < nit; ++it) {
-    const int buf = it & 1;
+  int cur_qi = is_qi;  // q tile index (within [0, ntq)) of iteration it
+  if (it_end > it_begin) issue(0);
+  for (int it = it_begin; it < it_end; ++it) {
+    const int buf = (it - it_begin) & 1;
     wait_vmcnt0();
     __syncthreads();
-    if (it + 1 < nit) issue(buf ^ 1);
+    if (it + 1 < it_end) issue(buf ^ 1);
     const int q0 = (qt_begin + cur_qi) * kDkvRows;
     if (++cur_qi == ntq) cur_qi = 0;
     const int q0_abs = p.q_offset + q0;
@@ -603,11 +632,79 @@ __global__ __launch_bounds__(kThreads, kBwdMinBlocks<DP>) void bwd_dkdv_kernel(c
     }
   }
 
+  if (cut) {
+    if (key < p.Skv) {
+      const int64_t tile = (static_cast<int64_t>(bh) * p.n_kt + kt) * p.n_part + part;
+      float* row = p.part + (tile * kDkvKeys + (key - k0)) * (D + Dv);
+#pragma unroll
+      for (int db = 0; db < S::DB; ++db) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int d0 = 32 * db + 8 * i + 4 * g;
+          const f32x4 k4 = {dkacc[db][4 * i], dkacc[db][4 * i + 1], dkacc[db][4 * i + 2],
+                            dkacc[db][4 * i + 3]};
+          if (d0 < D) *reinterpret_cast<f32x4*>(row + d0) = k4;
+          if (db < SV::DB) {
+            const f32x4 v4 = {dvacc[db][4 * i], dvacc[db][4 * i + 1], dvacc[db][4 * i + 2],
+                              dvacc[db][4 * i + 3]};
+            if (d0 < Dv) *reinterpret_cast<f32x4*>(row + D + d0) = v4;
+          }
+        }
+      }
+    }
+    return;
+  }
   if (wave_live && key < p.Skv) {
     store_rows<Tag, DP>(p.dk + b * p.dk_sb + hk * p.dk_sh + static_cast<int64_t>(key) * p.dk_ss,
                         dkacc, p.scale, D, g);
     store_rows<Tag, DV>(p.dv + b * p.dv_sb + hk * p.dv_sh + static_cast<int64_t>(key) * p.dv_ss,
                         dvacc, 1.0f, Dv, g);
+  }
+}
+
+// dK and dV of the key tiles whose sweep was cut: the sum of its parts in part order.
+// One thread per 4 dims of a key; grid (key tile, part of its rows).
+template <typename Tag>
+__global__ __launch_bounds__(kThreads) void bwd_dkdv_sum_kernel(const BwdParams p) {
+  using E = Elem<Tag>;
+  const int tile = blockIdx.x;  // (batch, KV head), key tile
+  const int bh = tile / p.n_kt;
+  const int kt = tile - bh * p.n_kt;
+  int first, n;
+  dkv_rows(p, kt, first, n);
+  const int nit = n * p.ratio;
+  if (nit <= p.part_len) return;
+  const int parts = (nit + p.part_len - 1) / p.part_len;
+  const int b = bh / p.Hkv;
+  const int hk = bh - b * p.Hkv;
+  const int width = p.D + p.Dv;  // multiples of 8
+  const int per_row = width >> 2;
+  const int keys = min(kDkvKeys, p.Skv - kt * kDkvKeys);
+  const float* base = p.part + static_cast<int64_t>(tile) * p.n_part * kDkvKeys * width;
+  for (int idx = blockIdx.y * kThreads + threadIdx.x; idx < keys * per_row; idx += gridDim.y * kThreads) {
+    const int r = idx / per_row;
+    const int d0 = 4 * (idx - r * per_row);
+    const float* src = base + static_cast<int64_t>(r) * width + d0;
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int i0 = 0; i0 < parts; i0 += 4) {
+      f32x4 x[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        x[u] = *reinterpret_cast<const f32x4*>(src + static_cast<int64_t>(min(i0 + u, parts - 1)) *
+                                                         kDkvKeys * width);
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        if (i0 + u < parts) acc += x[u];
+      }
+    }
+    const int64_t key = static_cast<int64_t>(kt) * kDkvKeys + r;
+    const bool is_k = d0 < p.D;
+    const float mul = is_k ? p.scale : 1.0f;
+    uint16_t* dst = is_k ? p.dk + b * p.dk_sb + hk * p.dk_sh + key * p.dk_ss + d0
+                         : p.dv + b * p.dv_sb + hk * p.dv_sh + key * p.dv_ss + (d0 - p.D);
+    *reinterpret_cast<u32x2*>(dst) =
+        u32x2{E::pack2(acc[0] * mul, acc[1] * mul), E::pack2(acc[2] * mul, acc[3] * mul)};
   }
 }
 
@@ -1463,7 +1560,17 @@ void launch_f32(const BwdParams& p, bool softcap, int grid_pre, hipStream_t s) {
 template <typename Tag, int DP, bool SOFTCAP, int DV = DP>
 void launch_main(const BwdParams& p, int grid_dkv, int grid_dq, hipStream_t s) {
   if (grid_dkv > 0) {
-    hipLaunchKernelGGL((bwd_dkdv_kernel<Tag, DP, DV, SOFTCAP>), dim3(grid_dkv), dim3(kThreads), 0, s, p);
+    bool cut = false;
+    if constexpr (DP <= kCutMaxDim) cut = p.n_part > 1;
+    if constexpr (DP <= kCutMaxDim) {
+      if (cut) {
+        hipLaunchKernelGGL((bwd_dkdv_kernel<Tag, DP, DV, SOFTCAP, true>), dim3(grid_dkv), dim3(kThreads), 0, s, p);
+        hipLaunchKernelGGL((bwd_dkdv_sum_kernel<Tag>), dim3(grid_dkv / p.n_part, 8), dim3(kThreads), 0, s, p);
+      }
+    }
+    if (!cut) {
+      hipLaunchKernelGGL((bwd_dkdv_kernel<Tag, DP, DV, SOFTCAP, false>), dim3(grid_dkv), dim3(kThreads), 0, s, p);
+    }
   }
   hipLaunchKernelGGL((bwd_dq_kernel<Tag, DP, DV, SOFTCAP>), dim3(grid_dq), dim3(kThreads), 0, s, p);
 }
@@ -1502,8 +1609,70 @@ size_t attn_bwd_workspace_bytes(int32_t batch, int32_t heads_q, int32_t seqlen_q
   return static_cast<size_t>(2) * batch * heads_q * sq_padded(seqlen_q) * sizeof(float);
 }
 
+namespace {
+
+// Cuts the dK/dV sweeps of a launch that its heaviest workgroup would hold up: sets n_part
+// and part_len, returns the bytes of the partials (0: no sweep is cut). A part is 1.5 times
+// an even share of the work over the chip's slots (two workgroups per CU up to head_dim
+// 128), at least 16 tiles; sweeps are cut when the longest exceeds 2.5 parts, so that the
+// partials (written and read once in fp32) cost less than the waiting. Measured on MI355X,
+// whole backward, bf16, us uncut / cut (B, Hq/Hkv, S, D, causal unless said):
+//   2, 32/8, 2011, 128    409 / 306      1, 40/8, 1024, 128, softcap   270 / 107
+//   1, 32/8, 4096, 128    774 / 555      1, 28/4, 1500, 96             432 / 146
+//   1, 8/8, 2048, 128     132 / 107      2, 8/1, 1000, 64              243 / 56
+//   1, 24/8, 2000, 192    373 / 223      1, 8/8, 4096, 64              180 / 150
+// with parts of one even share 1, 12/12, 2048, 128 not causal: 137 / 151, so it stays uncut.
+size_t plan_dkv_parts(BwdParams& p, int32_t dtype) {
+  p.n_part = 1;
+  p.part_len = 0x7fffffff;
+  const int64_t units = static_cast<int64_t>(p.B) * p.Hkv;
+  const int64_t slots = p.D <= 128 ? 512 : 256;
+  if (dtype == FFA_DTYPE_FP32 || p.D > kCutMaxDim || p.n_kt == 0 || units * p.n_kt >= 1024) return 0;
+  int64_t total = 0, most = 0;
+  for (int kt = 0; kt < p.n_kt; ++kt) {
+    int first, n;
+    dkv_rows(p, kt, first, n);
+    const int64_t nit = static_cast<int64_t>(n) * p.ratio;
+    total += nit;
+    most = nit > most ? nit : most;
+  }
+  int64_t len = (3 * total * units + 2 * slots - 1) / (2 * slots);
+  len = len < 16 ? 16 : len;
+  if (2 * most <= 5 * len) return 0;
+  if (most > 16 * len) len = (most + 15) / 16;  // at most 16 parts
+  p.n_part = static_cast<int>((most + len - 1) / len);
+  p.part_len = static_cast<int>(len);
+  return static_cast<size_t>(units) * p.n_kt * p.n_part * kDkvKeys * (p.D + p.Dv) * sizeof(float);
+}
+
+void fill_bwd_sizes(const ffa_attn_bwd_args& a, BwdParams& p) {
+  p.B = a.batch;
+  p.Hq = a.heads_q;
+  p.Hkv = a.heads_kv;
+  p.Sq = a.seqlen_q;
+  p.Skv = a.seqlen_kv;
+  p.D = a.head_dim;
+  p.Dv = a.v_head_dim > 0 ? a.v_head_dim : a.head_dim;
+  p.q_offset = a.q_offset;
+  p.causal = a.causal ? 1 : 0;
+  p.window = clamp_window(a.window, a.q_offset, a.seqlen_q);
+  p.ratio = a.heads_q / a.heads_kv;
+  p.sq_pad = static_cast<int>(sq_padded(a.seqlen_q));
+  p.n_qt = p.sq_pad / kQTile;
+  p.n_kt = (a.seqlen_kv + kDkvKeys - 1) / kDkvKeys;
+}
+
+}  // namespace
+
+size_t attn_bwd_split_workspace_bytes(const ffa_attn_bwd_args& a) {
+  BwdParams p{};
+  fill_bwd_sizes(a, p);
+  return attn_bwd_workspace_bytes(a.batch, a.heads_q, a.seqlen_q) + plan_dkv_parts(p, a.dtype);
+}
+
 int launch_attn_bwd(const ffa_attn_bwd_args& a, hipStream_t stream) {
   BwdParams p{};
+  fill_bwd_sizes(a, p);
   p.q = static_cast<const uint16_t*>(a.q);
   p.k = static_cast<const uint16_t*>(a.k);
   p.v = static_cast<const uint16_t*>(a.v);
@@ -1540,20 +1709,6 @@ int launch_attn_bwd(const ffa_attn_bwd_args& a, hipStream_t stream) {
   p.l_sb = a.lse_stride[0];
   p.l_sh = a.lse_stride[1];
   p.l_ss = a.lse_stride[2];
-  p.B = a.batch;
-  p.Hq = a.heads_q;
-  p.Hkv = a.heads_kv;
-  p.Sq = a.seqlen_q;
-  p.Skv = a.seqlen_kv;
-  p.D = a.head_dim;
-  p.Dv = a.v_head_dim > 0 ? a.v_head_dim : a.head_dim;
-  p.q_offset = a.q_offset;
-  p.causal = a.causal ? 1 : 0;
-  p.window = clamp_window(a.window, a.q_offset, a.seqlen_q);
-  p.ratio = a.heads_q / a.heads_kv;
-  p.sq_pad = static_cast<int>(sq_padded(a.seqlen_q));
-  p.n_qt = p.sq_pad / kQTile;
-  p.n_kt = (a.seqlen_kv + kDkvKeys - 1) / kDkvKeys;
   const bool softcap = a.softcap > 0.0f;
   if (softcap) {
     p.score_mul = a.scale / a.softcap;
@@ -1569,10 +1724,17 @@ int launch_attn_bwd(const ffa_attn_bwd_args& a, hipStream_t stream) {
   const int64_t rows = static_cast<int64_t>(a.batch) * a.heads_q * p.sq_pad;
   p.lse2 = ws;
   p.di = ws + rows;
+  const size_t stats = attn_bwd_workspace_bytes(a.batch, a.heads_q, a.seqlen_q);
+  const size_t parts = plan_dkv_parts(p, a.dtype);
+  p.part = ws + stats / sizeof(float);
+  if (parts == 0 || a.workspace_bytes < stats + parts) {
+    p.n_part = 1;
+    p.part_len = 0x7fffffff;
+  }
 
   const int64_t grid_pre = rows / 32;
   const int64_t grid_dq = static_cast<int64_t>(p.n_qt) * a.batch * a.heads_q;
-  const int64_t grid_dkv = static_cast<int64_t>(p.n_kt) * a.batch * a.heads_kv;
+  const int64_t grid_dkv = static_cast<int64_t>(p.n_kt) * p.n_part * a.batch * a.heads_kv;
   if (grid_pre > 0x7fffffff || grid_dq > 0x7fffffff || grid_dkv > 0x7fffffff) {
     return FFA_ERR_TOO_LARGE;
   }

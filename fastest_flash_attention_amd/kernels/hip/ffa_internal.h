@@ -37,6 +37,7 @@ int launch_mla_assemble(const ffa_mla_assemble_args& a, hipStream_t stream);
 
 // Attention backward: preprocess, dK/dV and dQ kernels.
 size_t attn_bwd_workspace_bytes(int32_t batch, int32_t heads_q, int32_t seqlen_q);
+size_t attn_bwd_split_workspace_bytes(const ffa_attn_bwd_args& a);
 int launch_attn_bwd(const ffa_attn_bwd_args& a, hipStream_t stream);
 
 // get_kv gather.

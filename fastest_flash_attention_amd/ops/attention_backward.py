@@ -16,6 +16,7 @@ not change the gradients, so it is accepted and ignored.
 
 from __future__ import annotations
 
+import ctypes
 import math
 from typing import Optional, Tuple
 
@@ -117,14 +118,10 @@ def fastest_flash_attn_backward(
         dv.zero_()
     else:
         lib = _lib.load()
-        ws_bytes = lib.ffa_attn_bwd_workspace_bytes(B, Hq, Sq)
-        ws = torch.empty((max(ws_bytes, 16) + 3) // 4, dtype=torch.float32, device=dev)
         a = _lib.AttnBwdArgs()
         a.dout, a.q, a.k, a.v, a.o = (t.data_ptr() for t in (do_c, q_c, k_c, v_c, o_c))
         a.lse = lse_c.data_ptr()
         a.dq, a.dk, a.dv = dq.data_ptr(), dk.data_ptr(), dv.data_ptr()
-        a.workspace = ws.data_ptr()
-        a.workspace_bytes = ws.numel() * 4
         a.do_stride[:] = list(do_c.stride())
         a.q_stride[:] = list(q_c.stride())
         a.k_stride[:] = list(k_c.stride())
@@ -143,6 +140,11 @@ def fastest_flash_attn_backward(
         a.softcap = float(softcap) if softcap is not None else 0.0
         a.dtype = code
         a.v_head_dim = Dv if narrow_v else 0
+        ws_bytes = max(lib.ffa_attn_bwd_split_workspace_bytes(ctypes.byref(a)),
+                       lib.ffa_attn_bwd_workspace_bytes(B, Hq, Sq), 16)
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+        a.workspace = ws.data_ptr()
+        a.workspace_bytes = ws_bytes
         _lib.launch(lib.ffa_attn_bwd, a, dev)
     if d_pad != D:
         dq, dk = (t[..., :D].contiguous() for t in (dq, dk))

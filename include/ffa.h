@@ -54,7 +54,7 @@
 extern "C" {
 #endif
 
-#define FFA_ABI_VERSION 10
+#define FFA_ABI_VERSION 11
 
 typedef enum ffa_status {
   FFA_OK = 0,
@@ -487,6 +487,10 @@ typedef struct ffa_attn_bwd_args {
 } ffa_attn_bwd_args;
 
 size_t ffa_attn_bwd_workspace_bytes(int32_t batch, int32_t heads_q, int32_t seqlen_q);
+/* Workspace of this call with which its dK/dV sweeps may be cut over more workgroups (few
+ * and uneven ones otherwise); >= ffa_attn_bwd_workspace_bytes, with which it runs too.
+ * Reads sizes and options only. 0 for sizes that ffa_attn_bwd refuses. */
+size_t ffa_attn_bwd_split_workspace_bytes(const ffa_attn_bwd_args* args);
 int ffa_attn_bwd(const ffa_attn_bwd_args* args, void* stream);
 
 const char* ffa_strerror(int status);
