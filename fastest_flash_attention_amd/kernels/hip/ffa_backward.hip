@@ -1427,8 +1427,13 @@ __global__ __launch_bounds__(kThreads, kF32mDqBlocks<DP>) void bwd_f32m_dq_kerne
   // heaviest row blocks (causal: the last) first, all heads at once
   const int units = p.B * p.Hq;
   const int n_rb = (p.Sq + kM32 - 1) / kM32;
-  const int jb = static_cast<int>(blockIdx.x) / units;
-  const int bh = static_cast<int>(blockIdx.x) - jb * units;
+  int rank = blockIdx.x;
+  const int n_items = units * n_rb;
+  if (kF32mDqBlocks<DP> == 2 && p.causal && n_items > 256 && n_items <= 512) {
+    rank = paired_rank(rank, 256, n_items);
+  }
+  const int jb = rank / units;
+  const int bh = rank - jb * units;
   const int rb = p.causal ? n_rb - 1 - jb : jb;
   const int b = bh / p.Hq;
   const int h = bh - b * p.Hq;

@@ -13,6 +13,17 @@
 
 namespace ffa {
 
+// Launches of 257 to 512 workgroups, two to a CU, are resident all at once: the second 256
+// join the first on their CUs in the same order, and nothing is left to even things out.
+// With the heaviest first throughout, the heaviest CU of a causal launch holds tile 0 and
+// the middle one; so the second 256 run lightest first (`n` items, `first` on the CUs
+// before the second round starts). On MI355X, causal, us before / after: fp32 forward B 2,
+// 8 heads, S 1024, D 64 38.5 / 33.8, B 1, 8, 2000 64.5 / 53.1 (their backward, dQ paired,
+// 111 / 106, 203 / 186); bf16 forward B 4, 8, 2048, D 128, softcap 57.5 / 53.7, without
+// 47.4 / 46.1, D 64 22.3 / 21.7. The bf16 backward kernels did not change.
+constexpr int paired_rank(int k, int first, int n) { return k < first ? k : n - 1 - (k - first); }
+constexpr int kPaired = 256;  // flag in xcd_group: pair the ranks of each XCD's 32 CUs
+
 // Prefill: grid = n_units * n_qt workgroups, unit = batch x q-head, jq = query tile
 // (jq = 0 is the heaviest causal tile). With xcd_group = G > 0 (needs n_units % 8 ==
 // 0), XCD x owns units [x HX, (x + 1) HX) (HX = n_units / 8) and runs them one after
@@ -25,7 +36,8 @@ constexpr void prefill_work_item(int bid, int grid, int n_qt, int xcd_group, int
   if (xcd_group > 0) {
     const int hx = (grid / n_qt) >> 3;
     const int x = bid & 7;
-    const int k = bid >> 3;
+    const int k = (xcd_group & kPaired) ? paired_rank(bid >> 3, 32, grid >> 3) : bid >> 3;
+    xcd_group &= kPaired - 1;
     const int gl = hx < xcd_group ? hx : xcd_group;
     const int k0 = (hx - gl) * n_qt;  // tiles of the units run one after another
     if (k < k0) {
@@ -55,11 +67,15 @@ constexpr void prefill_work_item(int bid, int grid, int n_qt, int xcd_group, int
 // cfg3 and +3.5 % at cfg5, the last four +1.5 % at cfg2 (-0.5 % at the north star,
 // all 16 there -2.6 %). Other grids that split evenly over the XCDs keep consecutive
 // ids on one XCD.
+// two_per_cu: the kernel runs two workgroups on a CU; then launches that fit the chip at
+// once pair their tiles (all units interleaved: tile rank = position), from eight tiles a
+// unit on (below that they differ too little: four tiles 22.7 / 23.1 us).
 constexpr void prefill_grid_order(bool causal, int64_t n_units, int64_t grid, int& xcd_group,
-                                  int& xcd_remap) {
+                                  int& xcd_remap, bool two_per_cu = false) {
   xcd_remap = (grid % 8 == 0) ? 1 : 0;
   const int64_t n_qt = n_units > 0 ? grid / n_units : 0;
   xcd_group = (causal && n_units % 8 == 0) ? (n_units / 8 <= 8 ? 8 : (n_qt <= 32 ? 4 : 2)) : 0;
+  if (two_per_cu && xcd_group == 8 && n_qt >= 8 && grid > 256 && grid <= 512) xcd_group |= kPaired;
 }
 
 // The backward's dK/dV and dQ grids (unit = batch x head, tile j = 0 the heaviest causal

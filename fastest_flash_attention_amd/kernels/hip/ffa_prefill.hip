@@ -1306,8 +1306,11 @@ __global__ __launch_bounds__(kThreads, kF32SplitBlocks<DP>) void prefill_f32_spl
   // heaviest row blocks (causal: the last) first, all heads at once
   const int units = p.B * p.Hq;
   const int n_rb = (p.Sq + kF32BN - 1) / kF32BN;
-  const int jb = static_cast<int>(blockIdx.x) / units;
-  const int bh = static_cast<int>(blockIdx.x) - jb * units;
+  int rank = blockIdx.x;
+  const int n = units * n_rb;
+  if (kF32SplitBlocks<DP> == 2 && p.causal && n > 256 && n <= 512) rank = paired_rank(rank, 256, n);
+  const int jb = rank / units;
+  const int bh = rank - jb * units;
   const int rb = p.causal ? n_rb - 1 - jb : jb;
   const int b = bh / p.Hq;
   const int h = bh - b * p.Hq;
@@ -1735,7 +1738,7 @@ int launch_prefill(const ffa_prefill_args& a, hipStream_t stream) {
   if (cached) return FFA_ERR_WORKSPACE;  // only the split kernel reads a cache in place
   const int grid = static_cast<int>(grid64);
   prefill_grid_order(p.causal != 0, static_cast<int64_t>(a.batch) * a.heads_q, grid,
-                     p.xcd_group, p.xcd_remap);
+                     p.xcd_group, p.xcd_remap, a.head_dim <= 192);
 
   if (a.dtype == FFA_DTYPE_BF16) {
     launch_tag<Bf16Tag>(p, softcap, grid, stream);
