@@ -20,12 +20,13 @@ import torch  # noqa: F401  (must load torch's HIP runtime before libffa.so)
 
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libffa.so")
 
-FFA_ABI_VERSION = 11
+FFA_ABI_VERSION = 12
 FFA_DTYPE_BF16 = 0
 FFA_DTYPE_FP16 = 1
 FFA_DTYPE_FP32 = 2
 FFA_NOALLOC_SCRATCH_BYTES = 64 << 20  # include/ffa.h
 FFA_SPLIT_MIN_KEYS = 2048  # include/ffa.h
+FFA_APPEND_HOST_PAGES = 480  # include/ffa.h
 
 _I64x4 = ctypes.c_int64 * 4
 _I64x3 = ctypes.c_int64 * 3
@@ -131,6 +132,8 @@ class PagedAppendArgs(ctypes.Structure):
         ("start", ctypes.c_int32),
         ("n_tokens", ctypes.c_int32),
         ("elem_bytes", ctypes.c_int32),
+        ("host_pages", ctypes.c_void_p),
+        ("n_host_pages", ctypes.c_int32),
     ]
 
 

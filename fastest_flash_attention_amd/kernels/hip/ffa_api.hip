@@ -252,7 +252,8 @@ int ffa_paged_append(const ffa_paged_append_args* a, void* stream) {
     return FFA_ERR_INVALID_ARG;
   }
   if (a->n_tokens == 0) return FFA_OK;
-  if (a->k_pages == nullptr || a->k_new == nullptr || a->page_table == nullptr) {
+  if (a->k_pages == nullptr || a->k_new == nullptr ||
+      (a->page_table == nullptr && a->host_pages == nullptr)) {
     return FFA_ERR_INVALID_ARG;
   }
   // V is optional (K-only pools), but then entirely
@@ -261,6 +262,11 @@ int ffa_paged_append(const ffa_paged_append_args* a, void* stream) {
     if (a->k_new_stride[i] < 0 || a->v_new_stride[i] < 0) return FFA_ERR_INVALID_ARG;
   }
   if (static_cast<int64_t>(a->start) + a->n_tokens > 0x7fffffff) return FFA_ERR_TOO_LARGE;
+  if (a->host_pages != nullptr) {
+    const int64_t need = (static_cast<int64_t>(a->start) + a->n_tokens - 1) / a->page_size -
+                         a->start / a->page_size + 1;
+    if (a->n_host_pages < need || a->n_host_pages > FFA_APPEND_HOST_PAGES) return FFA_ERR_INVALID_ARG;
+  }
   return ffa::launch_paged_append(*a, static_cast<hipStream_t>(stream));
 }
 

@@ -25,9 +25,11 @@ device reduction and a host sync.
 
 from __future__ import annotations
 
+import ctypes
 import math
 from typing import Optional, Sequence, Tuple
 
+import numpy as np
 import torch
 
 from ..kernels import _lib
@@ -45,6 +47,47 @@ def _auto_tokens_per_split(batch: int, heads_kv: int, max_len: int) -> int:
     while tps > 64 and batch * heads_kv * max(1, math.ceil(max_len / tps)) < 256:
         tps //= 2
     return tps
+
+
+def device_ints(values, device: torch.device) -> torch.Tensor:
+    """int32 tensor of ``values`` (a list or an int32 array) on ``device``. To a ROCm device
+    it goes through pinned memory, behind the work queued there, without waiting for it
+    (a captured stream keeps the waiting copy, which capture refuses)."""
+    t = torch.from_numpy(np.asarray(values, dtype=np.int32))
+    if device.type != "cuda" or t.numel() == 0 or torch.cuda.is_current_stream_capturing():
+        return t.to(device)
+    return t.pin_memory().to(device, non_blocking=True)
+
+
+def device_tables(tables: Sequence[Sequence[int]], lens: Sequence[int],
+                  device: torch.device) -> Tuple[torch.Tensor, torch.Tensor]:
+    """int32 ``[B, max_blocks]`` block tables (rows padded with 0) and int32 ``[B]`` lengths,
+    sent to ``device`` in one copy."""
+    n = len(tables)
+    width = max([1] + [len(t) for t in tables])
+    flat = np.zeros(n * width + n, dtype=np.int32)
+    for i, t in enumerate(tables):
+        flat[i * width:i * width + len(t)] = t
+    flat[n * width:] = lens
+    both = device_ints(flat, device)
+    return both[:n * width].view(n, width), both[n * width:]
+
+
+def set_append_pages(a: _lib.PagedAppendArgs, table: Sequence[int], start: int, n: int,
+                     page_size: int, device: torch.device):
+    """Give an append the pages its tokens go to: inside the launch, or (more than
+    FFA_APPEND_HOST_PAGES) as the whole table on the device. Returns what must outlive the
+    launch."""
+    first = start // page_size
+    ids = table[first:(start + n - 1) // page_size + 1]
+    if len(ids) <= _lib.FFA_APPEND_HOST_PAGES and not torch.cuda.is_current_stream_capturing():
+        keep = (ctypes.c_int32 * len(ids))(*ids)
+        a.host_pages = ctypes.addressof(keep)
+        a.n_host_pages = len(ids)
+    else:
+        keep = device_ints(table, device)
+        a.page_table = keep.data_ptr()
+    return keep
 
 
 def check_page_ids(block_tables: torch.Tensor, context_lens: torch.Tensor, page_size: int,
@@ -422,13 +465,13 @@ class PagedKVCache:
             kn = kn.contiguous()
         if vn.stride(-1) != 1:
             vn = vn.contiguous()
-        table = torch.tensor(seq["page_table"], dtype=torch.int32, device=self.k_pages.device)
         a = _lib.PagedAppendArgs()
+        keep = set_append_pages(a, seq["page_table"], start, kn.size(1), self.page_size,  # noqa: F841
+                                self.k_pages.device)
         a.k_pages = self.k_pages.data_ptr()
         a.v_pages = self.v_pages.data_ptr()
         a.k_new = kn.data_ptr()
         a.v_new = vn.data_ptr()
-        a.page_table = table.data_ptr()
         a.k_new_stride[:] = [kn.stride(0), kn.stride(1)]
         a.v_new_stride[:] = [vn.stride(0), vn.stride(1)]
         a.num_pages = self.max_pages
@@ -443,8 +486,7 @@ class PagedKVCache:
         _lib.launch(_lib.load().ffa_paged_append, a, self.k_pages.device)
 
     def _page_table_tensor(self, seq_id: int) -> torch.Tensor:
-        return torch.tensor(self.sequences[seq_id]["page_table"], dtype=torch.int32,
-                            device=self.k_pages.device)
+        return device_ints(self.sequences[seq_id]["page_table"], self.k_pages.device)
 
     def _get_kv_host(self, seq_id: int) -> Tuple[torch.Tensor, torch.Tensor]:
         """``get_kv`` of a pool in host memory (the constructor's default device): one
@@ -504,12 +546,7 @@ class PagedKVCache:
             seq = self.sequences.get(sid, {"page_table": [], "len": 0})
             tables.append(seq["page_table"])
             lens.append(seq["len"])
-        width = max([1] + [len(t) for t in tables])
-        bt = torch.zeros(len(tables), width, dtype=torch.int32)
-        for i, t in enumerate(tables):
-            if t:
-                bt[i, : len(t)] = torch.tensor(t, dtype=torch.int32)
-        return bt.to(device), torch.tensor(lens, dtype=torch.int32).to(device)
+        return device_tables(tables, lens, device)
 
     def decode(
         self,

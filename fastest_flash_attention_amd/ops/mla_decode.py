@@ -25,7 +25,7 @@ from typing import Optional, Sequence, Tuple
 import torch
 
 from ..kernels import _lib
-from .kv_cache import check_page_ids
+from .kv_cache import check_page_ids, device_tables, set_append_pages
 
 MLA_ROPE_DIM = 64
 MLA_LATENT_DIMS = (256, 512)
@@ -314,13 +314,13 @@ class MLALatentCache:
 
     def _append_device(self, seq: dict, start: int, rows: torch.Tensor) -> None:
         """One K-only ``ffa_paged_append`` launch (the pool seen as one KV head)."""
-        table = torch.tensor(seq["page_table"], dtype=torch.int32, device=self.pages.device)
         a = _lib.PagedAppendArgs()
+        keep = set_append_pages(a, seq["page_table"], start, rows.size(0), self.page_size,  # noqa: F841
+                                self.pages.device)
         a.k_pages = self.pages.data_ptr()
         a.v_pages = None
         a.k_new = rows.data_ptr()
         a.v_new = None
-        a.page_table = table.data_ptr()
         a.k_new_stride[:] = [rows.numel(), rows.stride(0)]
         a.v_new_stride[:] = [0, 0]
         a.num_pages = self.max_pages
@@ -341,13 +341,7 @@ class MLALatentCache:
         lengths of ``seq_ids``."""
         device = self.pages.device if device is None else torch.device(device)
         tables = [self.sequences.get(s, {"page_table": []})["page_table"] for s in seq_ids]
-        width = max([1] + [len(t) for t in tables])
-        bt = torch.zeros(len(tables), width, dtype=torch.int32)
-        for i, t in enumerate(tables):
-            if t:
-                bt[i, : len(t)] = torch.tensor(t, dtype=torch.int32)
-        lens = torch.tensor([self.seq_len(s) for s in seq_ids], dtype=torch.int32)
-        return bt.to(device), lens.to(device)
+        return device_tables(tables, [self.seq_len(s) for s in seq_ids], device)
 
     def decode(self, q: torch.Tensor, seq_ids: Sequence[int], *, scale: float,
                return_lse: bool = False) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:

@@ -54,7 +54,7 @@
 extern "C" {
 #endif
 
-#define FFA_ABI_VERSION 11
+#define FFA_ABI_VERSION 12
 
 typedef enum ffa_status {
   FFA_OK = 0,
@@ -259,7 +259,14 @@ typedef struct ffa_paged_append_args {
   int32_t start;              /* tokens already stored for the sequence */
   int32_t n_tokens;
   int32_t elem_bytes;         /* 2 or 4 */
+  /* The page ids from the host instead (page_table is then not read): host_pages[i] is the
+     page of tokens (start / page_size + i) * page_size onwards, copied into the launch.
+     n_host_pages covers every token and is at most FFA_APPEND_HOST_PAGES. */
+  const int32_t* host_pages;
+  int32_t n_host_pages;
 } ffa_paged_append_args;
+
+#define FFA_APPEND_HOST_PAGES 480
 
 int ffa_paged_append(const ffa_paged_append_args* args, void* stream);
 
