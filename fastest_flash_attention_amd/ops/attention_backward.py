@@ -76,13 +76,14 @@ def fastest_flash_attn_backward(
         raise ValueError(f"num heads {Hq} is not a multiple of kv heads {Hkv}")
     if Bk != B and Bk != 1:
         raise ValueError(f"k/v batch {Bk} does not match q batch {B}")
-    for name, t in (("grad_output", grad_output), ("q", q), ("k", k), ("v", v),
-                    ("output", output), ("lse", lse)):
-        if t.device.type != "cuda":
-            raise RuntimeError(
-                f"fastest_flash_attention_amd runs on ROCm GPU tensors only; {name} is on "
-                f"{t.device} (there is no CPU path)"
-            )
+    tensors = (grad_output, q, k, v, output, lse)
+    if not all(t.is_cuda for t in tensors):
+        for name, t in zip(("grad_output", "q", "k", "v", "output", "lse"), tensors):
+            if t.device.type != "cuda":
+                raise RuntimeError(
+                    f"fastest_flash_attention_amd runs on ROCm GPU tensors only; {name} is on "
+                    f"{t.device} (there is no CPU path)"
+                )
     dtype = q.dtype
     if not (k.dtype == v.dtype == output.dtype == grad_output.dtype == dtype):
         raise TypeError("grad_output, q, k, v and output must share one dtype")

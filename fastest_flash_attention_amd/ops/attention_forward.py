@@ -135,8 +135,11 @@ def _expand_block_mask_device(bm, r: "ResolvedForward", device, n_br: int, words
 
 
 def _conforms(t: torch.Tensor) -> bool:
-    return (t.stride(-1) == 1 and t.data_ptr() % 16 == 0
-            and all(st % 8 == 0 for st, n in zip(t.stride()[:3], t.shape[:3]) if n > 1))
+    b, h, s, d = t.stride()
+    if d != 1 or t.data_ptr() % 16:
+        return False
+    return (b | h | s) % 8 == 0 or all(
+        st % 8 == 0 for st, n in zip((b, h, s), t.shape[:3]) if n > 1)
 
 
 def _conform(t: torch.Tensor, d_pad: int) -> torch.Tensor:
@@ -322,13 +325,14 @@ def prepare_prefill(*args, out: Optional[torch.Tensor] = None, **kwargs) -> Pref
     """Resolve arguments, check device/dtype/features, allocate outputs, build the ABI
     struct. Launches nothing."""
     r = resolve_forward_args(*args, cache_in_place=True, **kwargs)
-    for name, t in (("q", r.q), ("k", r.k), ("v", r.v)):
-        if t.device.type != "cuda":
-            raise RuntimeError(
-                f"fastest_flash_attention_amd runs on ROCm GPU tensors only; {name} is on "
-                f"{t.device} (there is no CPU path)"
-            )
-    if not (r.q.device == r.k.device == r.v.device):
+    if not (r.q.is_cuda and r.k.is_cuda and r.v.is_cuda):
+        for name, t in (("q", r.q), ("k", r.k), ("v", r.v)):
+            if t.device.type != "cuda":
+                raise RuntimeError(
+                    f"fastest_flash_attention_amd runs on ROCm GPU tensors only; {name} is on "
+                    f"{t.device} (there is no CPU path)"
+                )
+    if not (r.q.get_device() == r.k.get_device() == r.v.get_device()):
         raise RuntimeError("q, k, v must be on the same device")
     if not (r.q.dtype == r.k.dtype == r.v.dtype):
         raise TypeError(f"q/k/v dtypes differ: {r.q.dtype}, {r.k.dtype}, {r.v.dtype}")

@@ -44,7 +44,7 @@ def _auto_tokens_per_split(batch: int, heads_kv: int, max_len: int) -> int:
     (B=64, 8 KV heads, lengths U[512, 32768]), +4% on 16 x 8k and 2 x 32k contexts
     (the latter with only 256 workgroups), -1% on 128 contexts of at most 2k tokens."""
     tps = 2048
-    while tps > 64 and batch * heads_kv * max(1, math.ceil(max_len / tps)) < 256:
+    while tps > 64 and batch * heads_kv * max(1, -(-max_len // tps)) < 256:
         tps //= 2
     return tps
 
@@ -232,13 +232,15 @@ def fastest_flash_paged_decode(
         max_context_len = int(context_lens.max().item()) if B > 0 else 0
     if block_tables.size(1) * page_size < max_context_len:
         raise ValueError("block_tables has fewer columns than max_context_len needs")
-    for name, t in (("q", q3), ("k_pages", k_pages), ("v_pages", v_pages),
-                    ("block_tables", block_tables), ("context_lens", context_lens)):
-        if t.device.type != "cuda":
-            raise RuntimeError(
-                f"fastest_flash_attention_amd paged decode runs on ROCm tensors only; "
-                f"{name} is on {t.device}"
-            )
+    if not (q3.is_cuda and k_pages.is_cuda and v_pages.is_cuda and block_tables.is_cuda
+            and context_lens.is_cuda):
+        for name, t in (("q", q3), ("k_pages", k_pages), ("v_pages", v_pages),
+                        ("block_tables", block_tables), ("context_lens", context_lens)):
+            if t.device.type != "cuda":
+                raise RuntimeError(
+                    f"fastest_flash_attention_amd paged decode runs on ROCm tensors only; "
+                    f"{name} is on {t.device}"
+                )
     if q3.dtype == torch.float32:
         out, lse = _paged_decode_fp32(q3, k_pages, v_pages, block_tables, context_lens,
                                       scale, softcap, sliding_window, return_lse,

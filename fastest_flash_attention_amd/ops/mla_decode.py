@@ -37,7 +37,7 @@ def _auto_mla_tokens_per_split(batch: int, head_groups: int, max_len: int) -> in
     batch 32, context 4096 this picks 512 tokens (34.4-35.8 us per step; 256 tokens with
     two workgroups per CU: 38.6 us; 1024 tokens, 128 workgroups: about 51 us)."""
     tps = 1024
-    while tps > 64 and batch * head_groups * max(1, math.ceil(max_len / tps)) < 256:
+    while tps > 64 and batch * head_groups * max(1, -(-max_len // tps)) < 256:
         tps //= 2
     return tps
 
@@ -97,11 +97,12 @@ def prepare_mla_decode(
     if dim_v not in MLA_LATENT_DIMS or dqk != dim_v + MLA_ROPE_DIM or dk != dqk:
         raise ValueError(f"MLA decode needs dim_v in {MLA_LATENT_DIMS} and rope dim "
                          f"{MLA_ROPE_DIM} (q last dim {dqk}, pages {dk}, dim_v {dim_v})")
-    for name, t in (("q", q), ("kv_pages", kv_pages), ("block_tables", block_tables),
-                    ("context_lens", context_lens)):
-        if t.device.type != "cuda":
-            raise RuntimeError(f"fastest_flash_attention_amd MLA decode runs on ROCm tensors "
-                               f"only; {name} is on {t.device}")
+    if not (q.is_cuda and kv_pages.is_cuda and block_tables.is_cuda and context_lens.is_cuda):
+        for name, t in (("q", q), ("kv_pages", kv_pages), ("block_tables", block_tables),
+                        ("context_lens", context_lens)):
+            if t.device.type != "cuda":
+                raise RuntimeError(f"fastest_flash_attention_amd MLA decode runs on ROCm tensors "
+                                   f"only; {name} is on {t.device}")
     if q.dtype != kv_pages.dtype:
         raise TypeError("q and kv_pages must share a dtype")
     code = _lib.dtype_code(q.dtype)
