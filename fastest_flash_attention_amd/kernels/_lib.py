@@ -20,7 +20,7 @@ import torch  # noqa: F401  (must load torch's HIP runtime before libffa.so)
 
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libffa.so")
 
-FFA_ABI_VERSION = 12
+FFA_ABI_VERSION = 13
 FFA_DTYPE_BF16 = 0
 FFA_DTYPE_FP16 = 1
 FFA_DTYPE_FP32 = 2
@@ -198,6 +198,20 @@ class MlaDecodeArgs(ctypes.Structure):
     ]
 
 
+class RopeTablesArgs(ctypes.Structure):
+    """Mirror of ``ffa_rope_tables_args``."""
+
+    _fields_ = [
+        ("inv_freq", ctypes.c_void_p),
+        ("cos", ctypes.c_void_p),
+        ("sin", ctypes.c_void_p),
+        ("seqlen", ctypes.c_int32),
+        ("half", ctypes.c_int32),
+        ("dtype", ctypes.c_int32),
+        ("table_dtype", ctypes.c_int32),
+    ]
+
+
 class MlaAssembleArgs(ctypes.Structure):
     """Mirror of ``ffa_mla_assemble_args``."""
 
@@ -285,6 +299,7 @@ EXPORTS = {
         [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32],
     ),
     "ffa_mla_decode_fwd": (ctypes.c_int, [ctypes.POINTER(MlaDecodeArgs), ctypes.c_void_p]),
+    "ffa_rope_tables": (ctypes.c_int, [ctypes.POINTER(RopeTablesArgs), ctypes.c_void_p]),
     "ffa_mla_assemble": (ctypes.c_int, [ctypes.POINTER(MlaAssembleArgs), ctypes.c_void_p]),
     "ffa_attn_bwd_workspace_bytes": (
         ctypes.c_size_t, [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32],

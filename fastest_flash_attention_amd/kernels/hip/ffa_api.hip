@@ -343,6 +343,22 @@ int ffa_mla_decode_fwd(const ffa_mla_decode_args* a, void* stream) {
   return ffa::launch_mla_decode(*a, static_cast<hipStream_t>(stream));
 }
 
+int ffa_rope_tables(const ffa_rope_tables_args* a, void* stream) {
+  if (a == nullptr) return FFA_ERR_INVALID_ARG;
+  if (!valid_dtype(a->dtype) || (a->table_dtype != a->dtype && a->table_dtype != FFA_DTYPE_FP32)) {
+    return FFA_ERR_UNSUPPORTED_DTYPE;
+  }
+  if (a->seqlen < 0 || a->half < 1) return FFA_ERR_INVALID_ARG;
+  if (a->seqlen == 0) return FFA_OK;
+  if (a->inv_freq == nullptr || a->cos == nullptr || a->sin == nullptr) return FFA_ERR_INVALID_ARG;
+  const uintptr_t unit = a->table_dtype == FFA_DTYPE_FP32 ? 4 : 2;
+  if (reinterpret_cast<uintptr_t>(a->inv_freq) % unit != 0 || reinterpret_cast<uintptr_t>(a->cos) % unit != 0 ||
+      reinterpret_cast<uintptr_t>(a->sin) % unit != 0) {
+    return FFA_ERR_MISALIGNED;
+  }
+  return ffa::launch_rope_tables(*a, static_cast<hipStream_t>(stream));
+}
+
 int ffa_mla_assemble(const ffa_mla_assemble_args* a, void* stream) {
   if (a == nullptr) return FFA_ERR_INVALID_ARG;
   if (!valid_dtype(a->dtype) || (a->table_dtype != a->dtype && a->table_dtype != FFA_DTYPE_FP32)) {

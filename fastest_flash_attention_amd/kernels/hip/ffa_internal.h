@@ -32,6 +32,9 @@ size_t mla_decode_workspace_bytes(int32_t batch, int32_t heads_q, int32_t dim_v,
                                   int32_t max_context_len, int32_t tokens_per_split);
 int launch_mla_decode(const ffa_mla_decode_args& a, hipStream_t stream);
 
+// RoPE cos / sin tables.
+int launch_rope_tables(const ffa_rope_tables_args& a, hipStream_t stream);
+
 // MLA queries and keys from the module's projections.
 int launch_mla_assemble(const ffa_mla_assemble_args& a, hipStream_t stream);
 

@@ -128,7 +128,52 @@ __global__ __launch_bounds__(256) void mla_assemble_kernel(const AssembleParams 
   }
 }
 
+// cos and sin of position * inv_freq, one entry per thread: four small elementwise launches
+// (positions, products, cos, sin) in one. Bound by launch latency: 5 us against 20 on MI355X
+// at 4096 positions of 32 frequencies, 1016 against 1034 us for the module's call there.
+template <typename Tag, bool TAB32>
+__global__ __launch_bounds__(256) void rope_tables_kernel(const ffa_rope_tables_args a) {
+#pragma clang fp contract(off)
+  using E = Elem<Tag>;
+  const int64_t id = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (id >= static_cast<int64_t>(a.seqlen) * a.half) return;
+  const int s = static_cast<int>(id / a.half);
+  const int i = static_cast<int>(id - static_cast<int64_t>(s) * a.half);
+  const float pos = as_table<Tag, false>(static_cast<float>(s));
+  if constexpr (TAB32) {
+    const float x = pos * static_cast<const float*>(a.inv_freq)[i];
+    static_cast<float*>(a.cos)[id] = cosf(x);
+    static_cast<float*>(a.sin)[id] = sinf(x);
+  } else {
+    const float x = as_table<Tag, false>(pos * E::to_f32(static_cast<const uint16_t*>(a.inv_freq)[i]));
+    const uint32_t both = E::pack2(cosf(x), sinf(x));
+    static_cast<uint16_t*>(a.cos)[id] = static_cast<uint16_t>(both & 0xffffu);
+    static_cast<uint16_t*>(a.sin)[id] = static_cast<uint16_t>(both >> 16);
+  }
+}
+
 }  // namespace
+
+int launch_rope_tables(const ffa_rope_tables_args& a, hipStream_t stream) {
+  const int64_t blocks = (static_cast<int64_t>(a.seqlen) * a.half + 255) / 256;
+  if (blocks > 0x7fffffff) return FFA_ERR_TOO_LARGE;
+  const dim3 grid(static_cast<unsigned>(blocks));
+  const bool tab32 = a.table_dtype == FFA_DTYPE_FP32;
+  if (a.dtype == FFA_DTYPE_BF16) {
+    if (tab32) {
+      hipLaunchKernelGGL((rope_tables_kernel<Bf16Tag, true>), grid, dim3(256), 0, stream, a);
+    } else {
+      hipLaunchKernelGGL((rope_tables_kernel<Bf16Tag, false>), grid, dim3(256), 0, stream, a);
+    }
+  } else {
+    if (tab32) {
+      hipLaunchKernelGGL((rope_tables_kernel<F16Tag, true>), grid, dim3(256), 0, stream, a);
+    } else {
+      hipLaunchKernelGGL((rope_tables_kernel<F16Tag, false>), grid, dim3(256), 0, stream, a);
+    }
+  }
+  return hipGetLastError() == hipSuccess ? FFA_OK : FFA_ERR_LAUNCH;
+}
 
 int launch_mla_assemble(const ffa_mla_assemble_args& a, hipStream_t stream) {
   AssembleParams p{};

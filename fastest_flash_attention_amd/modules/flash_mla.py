@@ -16,7 +16,7 @@ import torch.nn as nn
 
 from ..ops.attention_forward import forward_token_major, narrow_v
 from ..ops.attention_func import fastest_flash_attn_func
-from ..ops.mla_decode import MLALatentCache, mla_assemble, mla_assembles
+from ..ops.mla_decode import MLALatentCache, mla_assemble, mla_assembles, rope_tables
 
 
 def has_hooks(m: nn.Module) -> bool:
@@ -50,6 +50,9 @@ class RotaryEmbedding(nn.Module):
 
     def tables(self, x: torch.Tensor):
         """(cos, sin) ``[S, dim / 2]`` of ``forward(x)`` at offset 0, for x ``[B, S, *]``."""
+        tables = rope_tables(self.inv_freq, x)
+        if tables is not None:
+            return tables
         pos = torch.arange(x.size(1), device=x.device, dtype=x.dtype)
         freqs = torch.outer(pos, self.inv_freq.to(x.device))
         return freqs.cos(), freqs.sin()

@@ -204,6 +204,27 @@ def fastest_flash_mla_decode(
     return call.out, call.lse
 
 
+def rope_tables(inv_freq: torch.Tensor, x: torch.Tensor
+                ) -> Optional[Tuple[torch.Tensor, torch.Tensor]]:
+    """cos and sin ``[S, dim / 2]`` of x ``[B, S, *]``'s positions in one launch
+    (``ffa_rope_tables``: the values that the elementwise operations of these types give),
+    or None where it does not apply."""
+    if (not x.is_cuda or inv_freq.device != x.device or not inv_freq.is_contiguous()
+            or x.dtype not in (torch.bfloat16, torch.float16) or inv_freq.requires_grad
+            or inv_freq.dtype not in (x.dtype, torch.float32)):
+        return None
+    S, half = x.size(1), inv_freq.numel()
+    both = torch.empty(2, S, half, dtype=inv_freq.dtype, device=x.device)
+    cos, sin = both[0], both[1]
+    a = _lib.RopeTablesArgs()
+    a.inv_freq, a.cos, a.sin = inv_freq.data_ptr(), cos.data_ptr(), sin.data_ptr()
+    a.seqlen, a.half = S, half
+    a.dtype = _lib.dtype_code(x.dtype)
+    a.table_dtype = _lib.dtype_code(inv_freq.dtype, allow_fp32=True)
+    _lib.launch(_lib.load().ffa_rope_tables, a, x.device)
+    return cos, sin
+
+
 def mla_assembles(q_nope: torch.Tensor, q_rope: torch.Tensor, kv: torch.Tensor,
                   k_rope: torch.Tensor, head_dim: int, rope_dim: int) -> bool:
     """Whether ``mla_assemble`` takes these projections: plain 16-bit ROCm tensors of one

@@ -32,6 +32,7 @@
  *                              no MLA decode path; this one reads the compressed latent
  *                              cache instead of up-projected K/V.
  *   ffa_mla_decode_workspace_bytes: sizing helper of the MLA decode entry point.
+ *   ffa_rope_tables        <- RotaryEmbedding's cos and sin (modules/flash_mla.py:42-48).
  *   ffa_mla_assemble       <- q and k of FastestFlashMLA.forward (modules/flash_mla.py:
  *                             129-152): RoPE of the rope parts and the concatenations.
  *   ffa_attn_bwd           <- fastest_flash_attn_backward   ops/attention_backward.py:19-76
@@ -54,7 +55,7 @@
 extern "C" {
 #endif
 
-#define FFA_ABI_VERSION 12
+#define FFA_ABI_VERSION 13
 
 typedef enum ffa_status {
   FFA_OK = 0,
@@ -395,6 +396,24 @@ typedef struct ffa_mla_decode_args {
 size_t ffa_mla_decode_workspace_bytes(int32_t batch, int32_t heads_q, int32_t dim_v,
                                       int32_t max_context_len, int32_t tokens_per_split);
 int ffa_mla_decode_fwd(const ffa_mla_decode_args* args, void* stream);
+
+/*
+ * RoPE tables of positions 0 .. seqlen - 1: angle = position * inv_freq[i], cos and sin of
+ * it, each step rounded as elementwise operations of these types round it: the position to
+ * dtype, angle, cos and sin to table_dtype. inv_freq: [half] of table_dtype; cos, sin:
+ * contiguous [seqlen, half] of table_dtype.
+ */
+typedef struct ffa_rope_tables_args {
+  const void* inv_freq;
+  void* cos;
+  void* sin;
+  int32_t seqlen;
+  int32_t half;
+  int32_t dtype;        /* FFA_DTYPE_BF16 or FFA_DTYPE_FP16 */
+  int32_t table_dtype;  /* dtype or FFA_DTYPE_FP32 */
+} ffa_rope_tables_args;
+
+int ffa_rope_tables(const ffa_rope_tables_args* args, void* stream);
 
 /*
  * Queries and keys of the MLA module from its projections (modules/flash_mla.py:129-152):

@@ -125,3 +125,37 @@ def test_o_proj_without_the_zero_columns(B, S):
     assert calls == [(B, S, 2 * 192)]
     # bf16 outputs of one fp32 sum: at most a rounding of the last bit apart
     assert (got - whole).abs().max() <= 2 ** -7 * whole.abs().max()
+
+
+def test_rope_tables_abi_checks():
+    lib = _lib.load()
+
+    def rc(**kw):
+        a = _lib.RopeTablesArgs()
+        base = dict(inv_freq=16, cos=16, sin=16, seqlen=3, half=4, dtype=0, table_dtype=0)
+        for name, val in {**base, **kw}.items():
+            setattr(a, name, val)
+        return lib.ffa_rope_tables(ctypes.byref(a), None)
+
+    assert lib.ffa_rope_tables(None, None) == -1
+    assert rc(dtype=2) == -2 and rc(table_dtype=1) == -2
+    assert rc(seqlen=-1) == -1 and rc(half=0) == -1 and rc(sin=None) == -1
+    assert rc(cos=17) == -4 and rc(table_dtype=2, sin=18) == -4
+    assert rc(seqlen=0, cos=None) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", [BF16, F16])
+@pytest.mark.parametrize("table", [torch.float32, None])
+@pytest.mark.parametrize("S,R", [(1, 16), (77, 48), (4096, 64), (70000, 32)])
+def test_rope_tables_are_the_elementwise_ones(dt, table, S, R):
+    """Positions past fp16's range become infinities, and their tables NaN, in both."""
+    require_gpu()
+    say(f"rope tables S{S} R{R} {dt} {table}")
+    rope = flash_mla.RotaryEmbedding(R).cuda().to(table or dt)
+    x = torch.empty(1, S, 8, dtype=dt, device="cuda")
+    freqs = torch.outer(torch.arange(S, device="cuda", dtype=dt), rope.inv_freq)
+    for got, want in zip(rope.tables(x), (freqs.cos(), freqs.sin())):
+        assert got.dtype == want.dtype and got.is_contiguous()
+        assert torch.equal(got.isnan(), want.isnan())
+        assert torch.equal(got.nan_to_num(7.0), want.nan_to_num(7.0))
