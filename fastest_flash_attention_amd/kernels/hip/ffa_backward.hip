@@ -1264,16 +1264,19 @@ __device__ inline void store_acc_row_f32(float* row, const f32x16* acc, float mu
   }
 }
 
-// dK / dV: one workgroup per CU (its 4 waves hold K, V, dK and dV of 32 keys plus a
-// prefetched tile at head_dim 64; at 128 the tile is loaded when it is needed). dQ: two
-// per CU at head_dim 64.
+// dQ: two workgroups per CU at head_dim 64. dK / dV: one (its 4 waves hold K, V, dK and dV
+// of 32 keys plus a prefetched tile at head_dim 64; at 128 the tile is loaded when it is
+// needed), except at head_dim 64 with more than 384 workgroups: without the prefetched tile
+// and with its accumulators in VGPRs two fit (TWO: 245 registers), and the second hides more
+// than the prefetch did. On MI355X, whole backward, D 64, us one / two per CU: B 4, 16 heads,
+// S 1024 379 / 331, B 2, 8, 1024 103 / 98, B 1, 8, 2000 185 / 177, B 4, 8, 400 61 / 57; with
+// 384 workgroups (B 1, 12, 1024) 93 / 97, with 256 no difference.
 template <int DP>
 constexpr int kF32mDqBlocks = DP <= 64 ? 2 : 1;
-template <int DP>
-constexpr bool kF32mDkvPrefetch = DP <= 64;
+constexpr int64_t kF32mTwoFrom = 385;
 
-template <int DP, bool SOFTCAP>
-__global__ __launch_bounds__(kThreads, 1) void bwd_f32m_dkdv_kernel(const BwdParams p) {
+template <int DP, bool SOFTCAP, bool TWO>
+__global__ __launch_bounds__(kThreads, (TWO ? 2 : 1)) void bwd_f32m_dkdv_kernel(const BwdParams p) {
   using T = F32WaveTile<DP>;
   constexpr int PITCH = T::PITCH;
   constexpr int HALF = DP / 2;
@@ -1292,8 +1295,11 @@ __global__ __launch_bounds__(kThreads, 1) void bwd_f32m_dkdv_kernel(const BwdPar
 
   // heaviest key blocks (causal: block 0 sees every row) first, all heads at once
   const int units = p.B * p.Hkv;
-  const int kb = static_cast<int>(blockIdx.x) / units;
-  const int bh = static_cast<int>(blockIdx.x) - kb * units;
+  int rank = blockIdx.x;
+  const int n_all = units * ((p.Skv + kM32 - 1) / kM32);
+  if (TWO && p.causal && n_all <= 512) rank = paired_rank(rank, 256, n_all);
+  const int kb = rank / units;
+  const int bh = rank - kb * units;
   const int b = bh / p.Hkv;
   const int hk = bh - b * p.Hkv;
   const int D = p.D;
@@ -1323,7 +1329,7 @@ __global__ __launch_bounds__(kThreads, 1) void bwd_f32m_dkdv_kernel(const BwdPar
   for (int a = 0; a < 2 * DB; ++a) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[a][r] = 0.0f;
-    pin_agpr(acc[a]);
+    if constexpr (!TWO) pin_agpr(acc[a]);
   }
 
   T qn, dn;
@@ -1338,7 +1344,7 @@ __global__ __launch_bounds__(kThreads, 1) void bwd_f32m_dkdv_kernel(const BwdPar
     const int64_t ws = (static_cast<int64_t>(b) * p.Hq + hq) * p.sq_pad + q0 + l32;
     statn = (g == 0 ? p.lse2 : p.di)[ws];
   };
-  constexpr bool PREFETCH = kF32mDkvPrefetch<DP>;
+  constexpr bool PREFETCH = DP <= 64 && !TWO;
   if (PREFETCH && wave < n_items) fetch(wave);
   for (int i = wave; i < n_items; i += 4) {
     const int q0 = (j_lo + i % nj) * kM32;
@@ -1394,7 +1400,9 @@ __global__ __launch_bounds__(kThreads, 1) void bwd_f32m_dkdv_kernel(const BwdPar
       }
     }
 #pragma unroll
-    for (int a = 0; a < 2 * DB; ++a) pin_agpr(acc[a]);
+    for (int a = 0; a < 2 * DB; ++a) {
+      if constexpr (!TWO) pin_agpr(acc[a]);
+    }
     wave_lds_order();
   }
 
@@ -1546,7 +1554,16 @@ void launch_f32m_dp(const BwdParams& p, hipStream_t s) {
   const int grid_dkv = p.B * p.Hkv * ((p.Skv + kM32 - 1) / kM32);
   const int grid_dq = p.B * p.Hq * ((p.Sq + kM32 - 1) / kM32);
   if (grid_dkv > 0) {
-    hipLaunchKernelGGL((bwd_f32m_dkdv_kernel<DP, SOFTCAP>), dim3(grid_dkv), dim3(kThreads), 0, s, p);
+    bool two = false;
+    if constexpr (DP <= 64) {
+      two = grid_dkv >= kF32mTwoFrom;
+      if (two) {
+        hipLaunchKernelGGL((bwd_f32m_dkdv_kernel<DP, SOFTCAP, true>), dim3(grid_dkv), dim3(kThreads), 0, s, p);
+      }
+    }
+    if (!two) {
+      hipLaunchKernelGGL((bwd_f32m_dkdv_kernel<DP, SOFTCAP, false>), dim3(grid_dkv), dim3(kThreads), 0, s, p);
+    }
   }
   hipLaunchKernelGGL((bwd_f32m_dq_kernel<DP, SOFTCAP>), dim3(grid_dq), dim3(kThreads), 0, s, p);
 }

@@ -13,7 +13,7 @@ import fastest_flash_attention_amd as ffa
 from fastest_flash_attention_amd.kernels import _lib
 from oracle import reference_backward as rb
 from tests.gpu_util import np32, require_gpu, say, seeded
-from tests.test_gpu_backward import _check
+from tests.test_gpu_backward import _check, _oracle_forward
 
 BF16, F16 = torch.bfloat16, torch.float16
 
@@ -101,3 +101,23 @@ def test_cut_sweeps(B, Hq, Hkv, Sq, Skv, D, Dv, off, causal, window, softcap, dt
     ref = rb.backward(np32(do), np32(q), np32(k), np32(vp), np32(o), np32(lse), q_offset=off, **kw)
     for name, g, r in zip(("dq", "dk", "dv"), got, ref):
         _check(g, np.asarray(r)[..., :g.size(-1)], dt, name)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,H,S", [(3, 8, 512), (5, 7, 350), (4, 8, 401), (8, 8, 288)])
+@pytest.mark.parametrize("causal", [True, False])
+def test_fp32_workgroups_per_cu(B, H, S, causal):
+    """fp32 dK/dV at head_dim 64 around its switch to two workgroups per CU (384 blocks of 32
+    keys), inside the paired range (385 to 512) and past it."""
+    require_gpu()
+    dt = torch.float32
+    say(f"fp32 dkdv blocks {B * H * math.ceil(S / 32)} causal{causal}")
+    q, k, v, do = (seeded((B, H, S, 64), dt, i) for i in range(4))
+    kw = dict(causal=causal, scale=0.125)
+    o, lse = _oracle_forward(q, k, v, window=None, softcap=None, q_offset=0, **kw)
+    args = [torch.from_numpy(np.ascontiguousarray(x)).cuda() if isinstance(x, np.ndarray) else x.cuda()
+            for x in (do, q, k, v, o, lse)]
+    got = ffa.fastest_flash_attn_backward(*args, **kw)
+    ref = rb.backward(np32(do), np32(q), np32(k), np32(v), o, lse, **kw)
+    for name, g, r in zip(("dq", "dk", "dv"), got, ref):
+        _check(g, r, dt, name)
