@@ -116,7 +116,9 @@ def _expand_block_mask_device(bm, r: "ResolvedForward", device, n_br: int, words
     """``_expand_block_mask`` in one launch of ``ffa_block_mask_expand``. A host mask goes
     over through pinned memory, so the call does not wait for the work queued before it."""
     if bm.device.type == "cpu" and bm.numel() and not torch.cuda.is_current_stream_capturing():
-        bm = bm.contiguous().pin_memory().to(device, non_blocking=True)
+        # (always a copy: the caller may change its own, even pinned, mask after the call)
+        host = torch.empty(bm.shape, dtype=torch.bool, pin_memory=True)
+        bm = host.copy_(bm).to(device, non_blocking=True)
     else:
         bm = bm.to(device).contiguous()
     packed = torch.empty(n_br, words, dtype=torch.int64, device=device)

@@ -56,3 +56,19 @@ def test_same_as_the_elementwise_form(S_q, S_kv, bs, causal, window):
     for form in (bm, bm.cuda(), bm.t().contiguous().t().cuda(), bm.to(torch.float32), bm.numpy()):
         got, gw, gv = _expand_block_mask(form, r, device)
         assert gw == words and torch.equal(got.cpu(), want) and torch.equal(gv.cpu(), wv)
+
+
+@pytest.mark.gpu
+def test_a_pinned_mask_may_change_after_the_call():
+    require_gpu()
+    big = torch.randn(4096, 4096, device="cuda")
+    device = big.device
+    q = torch.zeros(1, 1, 640, 8)
+    bm = torch.ones(10, 10, dtype=torch.bool).pin_memory()
+    r = resolve_forward_args(q, q, q, block_size=64, block_mask=bm)
+    want, _, wv = _expand_block_mask(bm, r, torch.device("cpu"))
+    for _ in range(30):  # work queued ahead of the copy
+        big = big @ big * 1e-4
+    got, _, gv = _expand_block_mask(bm, r, device)
+    bm.zero_()
+    assert torch.equal(got.cpu(), want) and torch.equal(gv.cpu(), wv)
