@@ -113,8 +113,9 @@ class FastestFlashMLA(nn.Module):
         kv = self.kv_up_proj(self.kv_down_proj(x))
         k_rope = self.k_rope_proj(x)
         v = kv.view(B, S, H, 2 * self.head_dim).transpose(1, 2)[..., self.head_dim:]
-        if type(self.rope) is RotaryEmbedding and not has_hooks(self.rope) and mla_assembles(
-                q_nope, q_rope, kv, k_rope, self.head_dim, self.rope_dim):
+        if (type(self.rope) is RotaryEmbedding and not has_hooks(self.rope)
+                and 2 * self.rope.inv_freq.numel() == self.rope_dim
+                and mla_assembles(q_nope, q_rope, kv, k_rope, self.head_dim, self.rope_dim)):
             # no gradient to keep: rotation and concatenation in one kernel, the same bits
             q, k = mla_assemble(q_nope, q_rope, kv, k_rope, *self.rope.tables(x), H,
                                 self.head_dim, self.rope_dim)
@@ -166,7 +167,8 @@ class FastestFlashMLA(nn.Module):
             return None  # the kernel writes the zeros
         if rows < 4096 or type(o) is not nn.Linear or o.bias is not None or has_hooks(o):
             return None
-        if type(o.weight) is not nn.Parameter:
+        if (type(o.weight) is not nn.Parameter
+                or o.weight.shape[1] != self.num_heads * self.attn_dim):
             return None
         heads = o.weight.view(-1, self.num_heads, self.attn_dim)[:, :, : self.head_dim]
         return heads.reshape(-1, self.num_heads * self.head_dim)

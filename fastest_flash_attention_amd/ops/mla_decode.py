@@ -249,6 +249,10 @@ def mla_assemble(q_nope: torch.Tensor, q_rope: torch.Tensor, kv: torch.Tensor,
     ``[B, S, *]`` (``ffa_mla_assemble``): the rope parts rotated by the tables ``[S,
     rope_dim / 2]`` and concatenated to the others, in one kernel."""
     B, S, _ = q_nope.shape
+    if (tuple(cos.shape) != (S, rope_dim // 2) or sin.shape != cos.shape
+            or q_nope.shape[2] != heads * head_dim or q_rope.shape != (B, S, heads * rope_dim)
+            or kv.shape != (B, S, 2 * heads * head_dim) or k_rope.shape != (B, S, rope_dim)):
+        raise ValueError("projections or tables do not match heads, head_dim and rope_dim")
     q = torch.empty(B, heads, S, head_dim + rope_dim, dtype=q_nope.dtype, device=q_nope.device)
     k = torch.empty_like(q)
     cos, sin = cos.contiguous(), sin.contiguous()

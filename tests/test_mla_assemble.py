@@ -159,3 +159,20 @@ def test_rope_tables_are_the_elementwise_ones(dt, table, S, R):
         assert got.dtype == want.dtype and got.is_contiguous()
         assert torch.equal(got.isnan(), want.isnan())
         assert torch.equal(got.nan_to_num(7.0), want.nan_to_num(7.0))
+
+
+@pytest.mark.gpu
+def test_rotary_of_another_width_keeps_the_general_path():
+    """A replaced rotary module whose tables have another width is not read by the kernel."""
+    require_gpu()
+    torch.manual_seed(0)
+    m = ffa.FastestFlashMLA(64, 2, head_dim=16, latent_dim=32, rope_dim=32).cuda().to(BF16).eval()
+    m.rope = flash_mla.RotaryEmbedding(16).cuda().to(BF16)
+    x = seeded((1, 40, 64), BF16, 2).cuda()
+    with torch.no_grad():
+        with pytest.raises(ValueError):
+            mla_assemble(m.q_proj(x), m.q_rope_proj(x), m.kv_up_proj(m.kv_down_proj(x)),
+                         m.k_rope_proj(x), *m.rope.tables(x), 2, 16, 32)
+        got = m.project_qkv(x, pad_v=False)
+    for g, w in zip(got, general(m, x)):
+        assert torch.equal(g, w)
