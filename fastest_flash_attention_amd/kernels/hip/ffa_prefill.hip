@@ -961,7 +961,9 @@ __global__ __launch_bounds__((64 * NW), (kMinBlocks<DP, SOFTCAP> * 4 / NW)) void
 }
 
 // O = sum_s 2^(lse_s - max) O_s / sum_s 2^(lse_s - max) over the key ranges, in range
-// order. Each row takes D / 4 lanes of 16-byte reads (rounded up to a power of two).
+// order. Each row takes D / 4 lanes of 16-byte reads (rounded up to a power of two). On
+// MI355X 8 us for 16288 rows of four ranges at D 128 (33 MB, 4.2 TB/s), 4 us for 256 rows of
+// eight (the floor of a launch whose length, lse and partial reads follow one another).
 template <typename Tag>
 __global__ __launch_bounds__(256) void prefill_merge_kernel(const PrefillParams p, int log2_lanes) {
   using E = Elem<Tag>;
