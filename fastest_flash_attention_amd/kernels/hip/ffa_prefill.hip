@@ -878,7 +878,8 @@ __global__ __launch_bounds__((64 * NW), (kMinBlocks<DP, SOFTCAP> * 4 / NW)) void
   const float l_tot = wave_pair_sum(l_run);
   if constexpr (SPLIT) {
     // partial of row (b, head, query): O normalised by this range's sum, and its lse in
-    // log2 units (-inf, and O left unwritten, when the row sees none of the range)
+    // log2 units (-inf, and O left unwritten, when the row sees none of the range: its sum is
+    // 0 then; a NaN sum, from a NaN or infinite score, is a partial like any other)
     // (the row is worked out again from an opaque copy of the lane, rather than held in
     // registers through the sweep)
     int r = lane;
@@ -888,7 +889,7 @@ __global__ __launch_bounds__((64 * NW), (kMinBlocks<DP, SOFTCAP> * 4 / NW)) void
       const int hr = pack ? r / p.Sq : 0;
       const int64_t slot =
           ((static_cast<int64_t>(b) * p.Hq + h + hr) * p.Sq + (r - hr * p.Sq)) * sp.n_split + split;
-      if (l_tot > 0.0f) {
+      if (l_tot != 0.0f) {
         const float inv = 1.0f / l_tot;
         float* orow = sp.ws_o + slot * D;
 #pragma unroll
@@ -904,7 +905,7 @@ __global__ __launch_bounds__((64 * NW), (kMinBlocks<DP, SOFTCAP> * 4 / NW)) void
           }
         }
       }
-      if (g == 0) sp.ws_lse[slot] = l_tot > 0.0f ? m_run * c + fast_log2(l_tot) : kNegInf;
+      if (g == 0) sp.ws_lse[slot] = l_tot != 0.0f ? m_run * c + fast_log2(l_tot) : kNegInf;
     }
     return;
   }

@@ -248,6 +248,46 @@ def test_rows_without_a_visible_key():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("D,softcap", [(64, None), (128, None), (192, None), (128, 20.0)])
+@pytest.mark.parametrize("cached", [False, True])
+def test_not_a_number_reaches_the_output(D, softcap, cached):
+    """A NaN query or key makes the rows that see it NaN, whichever range it lies in, and no
+    other row: a range with a NaN sum is not one without a visible key."""
+    require_gpu()
+    say(f"split nan D{D} cap{softcap} cached{cached}")
+    B, Hq, Hkv, Sq, Skv = 1, 4, 2, 40, 2200
+    q = seeded((B, Hq, Sq, D), BF16, 1)
+    k, v = (seeded((B, Hkv, Skv, D), BF16, s) for s in (2, 3))
+    kw = dict(causal=False, num_kv_heads=Hkv, softcap=softcap)
+
+    def call(q, k):
+        if not cached:
+            assert af.prepare_prefill(q.cuda(), k.cuda(), v.cuda(), **kw).args.workspace
+            return ffa.fastest_flash_attn_forward(q.cuda(), k.cuda(), v.cuda(), **kw)[0].cpu()
+        cache = tuple(t[:, :, :-Sq].cuda() for t in (k, v))
+        own = tuple(t[:, :, -Sq:].cuda() for t in (k, v))
+        assert af.prepare_prefill(q.cuda(), *own, kv_cache=cache, **kw).args.k_cache
+        return ffa.fastest_flash_attn_forward(q.cuda(), *own, kv_cache=cache, **kw)[0].cpu()
+
+    clean = call(q, k)
+    assert not clean.isnan().any()
+    bad_q = q.clone()
+    bad_q[0, 3, 7, 5] = float("nan")
+    out = call(bad_q, k)
+    rows = torch.zeros(B, Hq, Sq, dtype=torch.bool)
+    rows[0, 3, 7] = True
+    assert out[rows].isnan().all() and not out[~rows].isnan().any()
+    # (the rows of a wave move their running maxima together, so P may round to bf16
+    # elsewhere: each p by 2^-8 of itself at most, O by 2^-8 max |v|, and as much when stored)
+    assert (out[~rows].float() - clean[~rows].float()).abs().max() <= 2 ** -7 * v.float().abs().max()
+    for at in (0, 1000, Skv - 1):  # the first range, one inside, the last key
+        bad_k = k.clone()
+        bad_k[0, 1, at, D - 1] = float("nan")
+        out = call(q, bad_k)
+        assert out[:, 2:].isnan().all() and torch.equal(out[:, :2], clean[:, :2])
+
+
+@pytest.mark.gpu
 def test_block_mask_sweep_longer_than_the_tile_list():
     """A workgroup whose sweep has more key tiles than its live-tile list holds (2048) visits
     every tile; too many workgroups here for the keys to be split."""
