@@ -117,7 +117,8 @@ class FastestFlashMLA(nn.Module):
                 and 2 * self.rope.inv_freq.numel() == self.rope_dim
                 and mla_assembles(q_nope, q_rope, kv, k_rope, self.head_dim, self.rope_dim)):
             # no gradient to keep: rotation and concatenation in one kernel, the same bits
-            q, k = mla_assemble(q_nope, q_rope, kv, k_rope, *self.rope.tables(x), H,
+            # (the tables in the projections' dtype, which autocast makes another than x's)
+            q, k = mla_assemble(q_nope, q_rope, kv, k_rope, *self.rope.tables(q_rope), H,
                                 self.head_dim, self.rope_dim)
         else:
             q_nope = q_nope.view(B, S, H, self.head_dim).transpose(1, 2)
@@ -160,7 +161,8 @@ class FastestFlashMLA(nn.Module):
         copied out of the weight (50 MB read, 33 MB written, at hidden 4096, 32 heads).
         On MI355X, us, whole against without padding: 268 / 194 at 8192 rows, 138 / 106 at
         4096, 88 / 82 at 2048, 24 / 34 at 256 (hidden 4096, 32 heads); 71 / 61 and 46 / 42
-        at 8192 and 4096 rows (hidden 2048, 16 heads), 30 / 31 at 2048."""
+        at 8192 and 4096 rows (hidden 2048, 16 heads), 30 / 31 at 2048. (A weight that is
+        not finite in a left-out column does not meet a zero then, so it gives no NaN.)"""
         o = self.o_proj
         rows = q.size(0) * q.size(2)
         if not narrow_v(self.head_dim, self.attn_dim, q.dtype) or self.attn_dim % 8 != 0:

@@ -176,3 +176,19 @@ def test_rotary_of_another_width_keeps_the_general_path():
         got = m.project_qkv(x, pad_v=False)
     for g, w in zip(got, general(m, x)):
         assert torch.equal(g, w)
+
+
+@pytest.mark.gpu
+def test_autocast_builds_the_tables_in_the_projections_dtype():
+    """fp32 input and weights under autocast: bf16 projections, whose positions past 256 round
+    as the elementwise operations round them."""
+    require_gpu()
+    torch.manual_seed(0)
+    m = ffa.FastestFlashMLA(96, 2, head_dim=128, latent_dim=64, rope_dim=64).cuda().eval()
+    x = seeded((2, 700, 96), torch.float32, 5).cuda()
+    with torch.autocast("cuda", dtype=BF16):
+        want = general(m, x)
+        with torch.no_grad():
+            got = m.project_qkv(x, pad_v=False)
+    for g, w in zip(got, want):
+        assert g.dtype == w.dtype == BF16 and torch.equal(g, w)
