@@ -57,6 +57,12 @@ class RotaryEmbedding(nn.Module):
         freqs = torch.outer(pos, self.inv_freq.to(x.device))
         return freqs.cos(), freqs.sin()
 
+    def has_plain_tables(self, dtype: torch.dtype) -> bool:
+        """Whether ``forward`` of a ``dtype`` tensor takes constant tables of dtype or fp32."""
+        f = self.inv_freq
+        return (type(f) is torch.Tensor and f.dtype in (dtype, torch.float32)
+                and not f.requires_grad and not torch._C._functorch.is_functorch_wrapped_tensor(f))
+
     def rotate_at(self, x: torch.Tensor, positions: Sequence[int]) -> torch.Tensor:
         """RoPE of one token per batch row: x ``[B, ..., D_rope]``, token of row b at
         ``positions[b]``. Bitwise the rotation ``forward`` applies at that position
@@ -115,6 +121,7 @@ class FastestFlashMLA(nn.Module):
         v = kv.view(B, S, H, 2 * self.head_dim).transpose(1, 2)[..., self.head_dim:]
         if (type(self.rope) is RotaryEmbedding and not has_hooks(self.rope)
                 and 2 * self.rope.inv_freq.numel() == self.rope_dim
+                and self.rope.has_plain_tables(q_rope.dtype)
                 and mla_assembles(q_nope, q_rope, kv, k_rope, self.head_dim, self.rope_dim)):
             # no gradient to keep: rotation and concatenation in one kernel, the same bits
             # (the tables in the projections' dtype, which autocast makes another than x's)

@@ -192,3 +192,21 @@ def test_autocast_builds_the_tables_in_the_projections_dtype():
             got = m.project_qkv(x, pad_v=False)
     for g, w in zip(got, want):
         assert g.dtype == w.dtype == BF16 and torch.equal(g, w)
+
+
+@pytest.mark.gpu
+def test_double_or_learned_frequencies_keep_the_general_path():
+    """The kernel takes tables of the projections' dtype or fp32, and gives no gradient."""
+    require_gpu()
+    torch.manual_seed(0)
+    m = ffa.FastestFlashMLA(64, 2, head_dim=16, latent_dim=32, rope_dim=16).cuda().to(BF16).eval()
+    m.requires_grad_(False)
+    x = seeded((1, 40, 64), BF16, 2).cuda()
+    m.rope = flash_mla.RotaryEmbedding(16).cuda().double()
+    want_q = torch.cat([m.q_proj(x).view(1, 40, 2, 16).transpose(1, 2),
+                        m.rope(m.q_rope_proj(x).view(1, 40, 2, 16).transpose(1, 2))], dim=-1)
+    assert torch.equal(m.project_qkv(x, pad_v=False)[0], want_q)
+    m.rope = flash_mla.RotaryEmbedding(16).cuda()
+    m.rope.inv_freq.requires_grad_()
+    q, k, v = m.project_qkv(x, pad_v=False)
+    assert q.requires_grad and k.requires_grad and not v.requires_grad
