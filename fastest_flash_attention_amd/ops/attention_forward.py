@@ -325,7 +325,8 @@ def build_prefill_args(
 
 def prepare_prefill(*args, out: Optional[torch.Tensor] = None, **kwargs) -> PrefillCall:
     """Resolve arguments, check device/dtype/features, allocate outputs, build the ABI
-    struct. Launches nothing."""
+    struct. Starts no attention kernel; the launch reads q, k, v and a KV cache kept apart as
+    they are then."""
     r = resolve_forward_args(*args, cache_in_place=True, **kwargs)
     if not (r.q.is_cuda and r.k.is_cuda and r.v.is_cuda):
         for name, t in (("q", r.q), ("k", r.k), ("v", r.v)):
