@@ -19,9 +19,15 @@ from ..ops.attention_func import fastest_flash_attn_func
 from ..ops.mla_decode import MLALatentCache, mla_assemble, mla_assembles, rope_tables
 
 
-def has_hooks(m: nn.Module) -> bool:
-    return bool(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
-                or m._backward_pre_hooks or nn.modules.module._has_any_global_hook())
+def runs_only(m: nn.Module, cls: type) -> bool:
+    """Whether a call of ``m`` is ``cls.forward`` as its module defines it and nothing else,
+    so that its work may be done without the call: no subclass, no hook, no forward set on
+    the instance or the class (as offloading, adapter and quantisation wrappers set it)."""
+    hooks = (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
+             or m._backward_pre_hooks or nn.modules.module._has_any_global_hook())
+    own = getattr(cls.forward, "__globals__", {}).get("__name__") == cls.__module__
+    replaced = {"forward", "_call_impl", "_compiled_call_impl"} & vars(m).keys()
+    return type(m) is cls and own and not replaced and not hooks
 
 
 class RotaryEmbedding(nn.Module):
@@ -119,7 +125,7 @@ class FastestFlashMLA(nn.Module):
         kv = self.kv_up_proj(self.kv_down_proj(x))
         k_rope = self.k_rope_proj(x)
         v = kv.view(B, S, H, 2 * self.head_dim).transpose(1, 2)[..., self.head_dim:]
-        if (type(self.rope) is RotaryEmbedding and not has_hooks(self.rope)
+        if (runs_only(self.rope, RotaryEmbedding)
                 and 2 * self.rope.inv_freq.numel() == self.rope_dim
                 and self.rope.has_plain_tables(q_rope.dtype)
                 and mla_assembles(q_nope, q_rope, kv, k_rope, self.head_dim, self.rope_dim)):
@@ -174,7 +180,7 @@ class FastestFlashMLA(nn.Module):
         rows = q.size(0) * q.size(2)
         if not narrow_v(self.head_dim, self.attn_dim, q.dtype) or self.attn_dim % 8 != 0:
             return None  # the kernel writes the zeros
-        if rows < 4096 or type(o) is not nn.Linear or o.bias is not None or has_hooks(o):
+        if rows < 4096 or not runs_only(o, nn.Linear) or o.bias is not None:
             return None
         if (type(o.weight) is not nn.Parameter
                 or o.weight.shape[1] != self.num_heads * self.attn_dim):

@@ -45,6 +45,49 @@ def test_cpu_and_differentiable_inputs_take_the_general_path():
     assert q.requires_grad and k.requires_grad and v.requires_grad
 
 
+def replace_instance(m, forward, monkeypatch):
+    m.forward = lambda *args: forward(m, *args)
+
+
+def replace_class(m, forward, monkeypatch):
+    monkeypatch.setattr(type(m), "forward", lambda self, *args: forward(self, *args))
+
+
+def replace_compiled(m, forward, monkeypatch):
+    m._compiled_call_impl = lambda *args: forward(m, *args)
+
+
+@pytest.mark.parametrize("replace", [replace_instance, replace_class, replace_compiled])
+@pytest.mark.parametrize("name", ["o_proj", "rope"])
+def test_a_replaced_forward_is_called(name, replace, monkeypatch):
+    """A submodule whose forward was set from outside (by a wrapper that offloads, adapts or
+    quantises it) is called, also where the work of a plain one is done without the call: the
+    projection from 4096 rows on, the rotary module without gradients."""
+    m = ffa.FastestFlashMLA(64, 2, head_dim=128, latent_dim=32, rope_dim=64).to(BF16).eval()
+    seen, fused = [], []
+    monkeypatch.setattr(flash_mla, "mla_assembles", lambda *args: True)
+
+    def assemble(q_nope, q_rope, kv, k_rope, cos, sin, heads, head_dim, rope_dim):
+        fused.append("rope")
+        return (q_nope.new_zeros(1, heads, q_nope.size(1), head_dim + rope_dim),) * 2
+
+    def attend(q, k, v, drop_zero_dims=False, **kw):
+        fused.extend(["o_proj"] if drop_zero_dims else [])
+        return q.new_zeros(1, q.size(2), 2, 128 if drop_zero_dims else 192), None
+
+    monkeypatch.setattr(flash_mla, "mla_assemble", assemble)
+    monkeypatch.setattr(flash_mla, "forward_token_major", attend)
+    x = torch.zeros(1, 4096, 64, dtype=BF16)
+    with torch.no_grad():
+        m(x)
+        assert fused == ["rope", "o_proj"]  # a plain module
+        sub = getattr(m, name)
+        original = type(sub).forward
+        replace(sub, lambda mod, *args: (seen.append(mod), original(mod, *args))[1], monkeypatch)
+        m(x)
+    assert any(mod is sub for mod in seen) and fused.count(name) == 1
+
+
 def general(m, x):
     """project_qkv with the elementwise operations (the path of differentiable inputs)."""
     with torch.enable_grad():
