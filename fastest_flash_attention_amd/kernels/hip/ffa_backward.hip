@@ -86,9 +86,10 @@ struct BwdParams {
   int xcd_remap_dq, xcd_remap_dkv;
   int xcd_group_dq, xcd_group_dkv;  // > 0: units per interleaved group on one XCD
   int Dv;  // V's (and dV's) head dim, <= D: V is taken as zero-padded to D
-  // dK/dV sweeps cut into parts of part_len tiles, at most n_part of them (1: none is cut)
-  int n_part, part_len;
-  float* part;  // [B * Hkv][n_kt][n_part][128 keys][D + Dv] fp32 dK | dV of cut sweeps
+  // dK/dV sweeps cut into parts of part_len tiles, at most n_part of them (1: none is cut);
+  // those of key tiles [cut_first, cut_first + n_cut)
+  int n_part, part_len, cut_first, n_cut;
+  float* part;  // [B * Hkv][n_cut][n_part][128 keys][D + Dv] fp32 dK | dV of cut sweeps
 };
 
 constexpr int kCutMaxDim = 192;  // head_dim up to which dK/dV sweeps can be cut
@@ -634,7 +635,7 @@ __global__ __launch_bounds__(kThreads, kBwdMinBlocks<DP>) void bwd_dkdv_kernel(c
 
   if (cut) {
     if (key < p.Skv) {
-      const int64_t tile = (static_cast<int64_t>(bh) * p.n_kt + kt) * p.n_part + part;
+      const int64_t tile = (static_cast<int64_t>(bh) * p.n_cut + (kt - p.cut_first)) * p.n_part + part;
       float* row = p.part + (tile * kDkvKeys + (key - k0)) * (D + Dv);
 #pragma unroll
       for (int db = 0; db < S::DB; ++db) {
@@ -663,15 +664,15 @@ __global__ __launch_bounds__(kThreads, kBwdMinBlocks<DP>) void bwd_dkdv_kernel(c
 }
 
 // dK and dV of the key tiles whose sweep was cut: the sum of its parts in part order.
-// One thread per 4 dims of a key; grid (key tile, part of its rows). Bound by HBM: 13 us on
+// One thread per 4 dims of a key; grid (cut key tile, part of its rows). Bound by HBM: 13 us on
 // MI355X at B 2, 32/8 heads, S 2011, D 128 (three parts at most, 4 TB/s), beside 200 us of
 // the cut kernel and 317 of the uncut one.
 template <typename Tag>
 __global__ __launch_bounds__(kThreads) void bwd_dkdv_sum_kernel(const BwdParams p) {
   using E = Elem<Tag>;
-  const int tile = blockIdx.x;  // (batch, KV head), key tile
-  const int bh = tile / p.n_kt;
-  const int kt = tile - bh * p.n_kt;
+  const int tile = blockIdx.x;  // (batch, KV head), cut key tile
+  const int bh = tile / p.n_cut;
+  const int kt = p.cut_first + tile - bh * p.n_cut;
   int first, n;
   dkv_rows(p, kt, first, n);
   const int nit = n * p.ratio;
@@ -1589,7 +1590,7 @@ void launch_main(const BwdParams& p, int grid_dkv, int grid_dq, hipStream_t s) {
     if constexpr (DP <= kCutMaxDim) {
       if (cut) {
         hipLaunchKernelGGL((bwd_dkdv_kernel<Tag, DP, DV, SOFTCAP, true>), dim3(grid_dkv), dim3(kThreads), 0, s, p);
-        hipLaunchKernelGGL((bwd_dkdv_sum_kernel<Tag>), dim3(grid_dkv / p.n_part, 8), dim3(kThreads), 0, s, p);
+        hipLaunchKernelGGL((bwd_dkdv_sum_kernel<Tag>), dim3(p.B * p.Hkv * p.n_cut, 8), dim3(kThreads), 0, s, p);
       }
     }
     if (!cut) {
@@ -1635,8 +1636,8 @@ size_t attn_bwd_workspace_bytes(int32_t batch, int32_t heads_q, int32_t seqlen_q
 
 namespace {
 
-// Cuts the dK/dV sweeps of a launch that its heaviest workgroup would hold up: sets n_part
-// and part_len, returns the bytes of the partials (0: no sweep is cut). A part is 1.5 times
+// Cuts the dK/dV sweeps of a launch that its heaviest workgroup would hold up: sets n_part,
+// part_len and the key tiles cut, returns the bytes of the partials (0: no sweep is cut). A part is 1.5 times
 // an even share of the work over the chip's slots (two workgroups per CU up to head_dim
 // 128), at least 16 tiles; sweeps are cut when the longest exceeds 2.5 parts, so that the
 // partials (written and read once in fp32) cost less than the waiting. Measured on MI355X,
@@ -1666,7 +1667,22 @@ size_t plan_dkv_parts(BwdParams& p, int32_t dtype) {
   if (most > 16 * len) len = (most + 15) / 16;  // at most 16 parts
   p.n_part = static_cast<int>((most + len - 1) / len);
   p.part_len = static_cast<int>(len);
-  return static_cast<size_t>(units) * p.n_kt * p.n_part * kDkvKeys * (p.D + p.Dv) * sizeof(float);
+  // Only the key tiles with longer sweeps than a part have partials. A sweep's length is a
+  // concave function of the key tile (q_hi - q_lo of dkv_rows), so they follow one another
+  // and average at least (len + most) / 2: with len at least 1.5 even shares that is at most
+  // 4/3 slots partial tiles, 90 MB at head_dim 128 (683 of 128 KB), whatever the lengths
+  // of the sequences.
+  int end = 0;
+  p.cut_first = p.n_kt;
+  for (int kt = 0; kt < p.n_kt; ++kt) {
+    int first, n;
+    dkv_rows(p, kt, first, n);
+    if (static_cast<int64_t>(n) * p.ratio <= len) continue;
+    p.cut_first = kt < p.cut_first ? kt : p.cut_first;
+    end = kt + 1;
+  }
+  p.n_cut = end - p.cut_first;
+  return static_cast<size_t>(units) * p.n_cut * p.n_part * kDkvKeys * (p.D + p.Dv) * sizeof(float);
 }
 
 void fill_bwd_sizes(const ffa_attn_bwd_args& a, BwdParams& p) {

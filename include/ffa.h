@@ -514,7 +514,8 @@ typedef struct ffa_attn_bwd_args {
 
 size_t ffa_attn_bwd_workspace_bytes(int32_t batch, int32_t heads_q, int32_t seqlen_q);
 /* Workspace of this call with which its dK/dV sweeps may be cut over more workgroups (few
- * and uneven ones otherwise); >= ffa_attn_bwd_workspace_bytes, with which it runs too.
+ * and uneven ones otherwise); at least ffa_attn_bwd_workspace_bytes, with which it runs too,
+ * and at most 90 MB more.
  * Reads sizes and options only. 0 for sizes that ffa_attn_bwd refuses. */
 size_t ffa_attn_bwd_split_workspace_bytes(const ffa_attn_bwd_args* args);
 int ffa_attn_bwd(const ffa_attn_bwd_args* args, void* stream);

@@ -35,7 +35,7 @@ def test_workspace_query():
         return lib.ffa_attn_bwd_split_workspace_bytes(ctypes.byref(a)) - base
 
     n = extra(2, 32, 8, 2011, 2011, 128)
-    assert n > 0 and n % (2 * 8 * 16 * 128 * 256 * 4) == 0
+    assert n > 0 and n % (2 * 8 * 128 * 256 * 4) == 0
     assert extra(2, 32, 8, 2011, 2011, 192, Dv=128) % (128 * 320 * 4) == 0
     for plain in ((4, 32, 32, 8192, 8192, 128), (1, 2, 2, 100, 100, 64), (1, 8, 2, 2048, 2048, 256)):
         assert extra(*plain) == 0, plain
@@ -43,6 +43,25 @@ def test_workspace_query():
     assert extra(1, 8, 2, 2000, 0, 128) == 0
     assert lib.ffa_attn_bwd_split_workspace_bytes(None) == 0
     assert lib.ffa_attn_bwd_split_workspace_bytes(ctypes.byref(_args(1, 7, 2, 9, 9, 64))) == 0
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Skv,D,off,causal,window,tiles", [
+    # key tiles that see rows: a window's ten or so, the first sixteen of a prefix
+    (1, 32, 8, 512, 16000, 128, 15488, 1, 1024, 12),
+    (1, 8, 1, 2048, 65536, 128, 0, 1, 0, 16),
+    (1, 32, 1, 512, 130000, 128, 129488, 1, 1024, 13),
+    (1, 64, 2, 324, 63064, 192, 0, 1, 127, 3),
+    (3, 32, 1, 525, 32016, 192, 12526, 1, 102, 6),
+])
+def test_workspace_of_few_live_key_tiles(B, Hq, Hkv, Sq, Skv, D, off, causal, window, tiles):
+    """Partial tiles for the key tiles whose sweep is cut, at most sixteen each, and never more
+    than 4/3 of the workgroups that run at once."""
+    lib = _lib.load()
+    a = _args(B, Hq, Hkv, Sq, Skv, D, 0, off, causal, window)
+    extra = (lib.ffa_attn_bwd_split_workspace_bytes(ctypes.byref(a))
+             - lib.ffa_attn_bwd_workspace_bytes(B, Hq, Sq))
+    n, rest = divmod(extra, 128 * 2 * D * 4)
+    assert rest == 0 and 0 < n <= min(B * Hkv * tiles * 16, (512 if D <= 128 else 256) * 4 // 3)
 
 
 CASES = [
@@ -56,6 +75,9 @@ CASES = [
     (1, 8, 1, 800, 800, 192, 192, 0, True, None, None, BF16),
     (1, 4, 1, 900, 900, 192, 128, 0, True, None, None, BF16),   # V narrower than head_dim
     (1, 4, 1, 900, 900, 176, 72, 0, True, 500, None, F16),
+    # cut key tiles that start late and end early (two KV heads: their partials are adjacent)
+    (2, 16, 2, 260, 2500, 128, 128, 1900, True, 300, None, BF16),
+    (1, 16, 2, 500, 3000, 64, 64, 0, True, None, 20.0, F16),
 ]
 
 
