@@ -25,9 +25,9 @@ __global__ __launch_bounds__(256) void block_mask_expand_kernel(const ffa_block_
 
   for (int w = tid; w < a.words; w += 256) {
     const int k0 = 64 * w;
-    const int k1 = min(k0 + 64, Skv);  // keys past the end stay clear
+    const int k1 = min(k0 + 64, Skv);  // keys past the end, and words of only such, stay clear
     uint64_t bits = 0;
-    for (int j = k0 / bkv; j < n_bc && j * bkv < k1; ++j) {
+    for (int j = k0 / bkv; k0 < Skv && j < n_bc && j * bkv < k1; ++j) {
       if (row[j] == 0) continue;
       const int lo = max(j * bkv, k0) - k0;
       const int n = min((j + 1) * bkv, k1) - k0 - lo;

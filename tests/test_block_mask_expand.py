@@ -59,6 +59,27 @@ def test_same_as_the_elementwise_form(S_q, S_kv, bs, causal, window):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("S_kv,bkv,words", [(130, 100, 4), (64, 48, 3), (130, 64, 5), (65, 200, 300)])
+def test_words_past_the_last_key_are_clear(S_kv, bkv, words):
+    """The C entry takes more words than the keys need; the last tile, which may end in one of
+    them, sets no bit there."""
+    require_gpu()
+    say(f"mask words Skv{S_kv} bkv{bkv} words{words}")
+    n_bc = math.ceil(S_kv / bkv)
+    mask = torch.ones(2, n_bc, dtype=torch.bool, device="cuda")
+    bits = torch.full((2, words), -1, dtype=torch.int64, device="cuda")
+    visited = torch.empty(2, dtype=torch.int32, device="cuda")
+    a = _lib.BlockMaskArgs()
+    a.mask, a.key_mask, a.visited = mask.data_ptr(), bits.data_ptr(), visited.data_ptr()
+    a.mask_stride, a.words, a.seqlen_q, a.seqlen_kv = n_bc, words, 20, S_kv
+    a.block_q, a.block_kv = 16, bkv
+    _lib.launch(_lib.load().ffa_block_mask_expand, a, mask.device)
+    keys = torch.arange(words * 64).view(words, 64) < S_kv
+    want = (keys.to(torch.int64) << torch.arange(64)).sum(-1)
+    assert torch.equal(bits.cpu(), want.expand(2, -1)) and visited.tolist() == [n_bc, n_bc]
+
+
+@pytest.mark.gpu
 def test_a_pinned_mask_may_change_after_the_call():
     require_gpu()
     big = torch.randn(4096, 4096, device="cuda")
