@@ -24,6 +24,15 @@ namespace ffa {
 constexpr int paired_rank(int k, int first, int n) { return k < first ? k : n - 1 - (k - first); }
 constexpr int kPaired = 256;  // flag in xcd_group: pair the ranks of each XCD's 32 CUs
 
+// Whether a 16-bit prefill launch may pair its tiles. Not at head_dim 32 (three workgroups
+// on a CU), whose launches it slows: 1-4 % at every size without softcap (8 heads, S 8192
+// 68.9 / 72.0 us; 32, 2048 21.2 / 21.7), with softcap by up to 1.5 % to 384 workgroups (8,
+// S 5120 71.1 / 72.1); past them it gains 4-15 % there (8, S 8192 130 / 113). head_dim 64
+// without softcap, also three on a CU, gains up to 4 % (64, 1024 17.5 / 16.8).
+constexpr bool prefill_pairs(int head_dim, bool softcap, int64_t grid) {
+  return head_dim > 32 ? head_dim <= 192 : softcap && grid > 384;
+}
+
 // Prefill: grid = n_units * n_qt workgroups, unit = batch x q-head, jq = query tile
 // (jq = 0 is the heaviest causal tile). With xcd_group = G > 0 (needs n_units % 8 ==
 // 0), XCD x owns units [x HX, (x + 1) HX) (HX = n_units / 8) and runs them one after

@@ -1741,7 +1741,7 @@ int launch_prefill(const ffa_prefill_args& a, hipStream_t stream) {
   if (cached) return FFA_ERR_WORKSPACE;  // only the split kernel reads a cache in place
   const int grid = static_cast<int>(grid64);
   prefill_grid_order(p.causal != 0, static_cast<int64_t>(a.batch) * a.heads_q, grid,
-                     p.xcd_group, p.xcd_remap, a.head_dim <= 192);
+                     p.xcd_group, p.xcd_remap, prefill_pairs(a.head_dim, softcap, grid));
 
   if (a.dtype == FFA_DTYPE_BF16) {
     launch_tag<Bf16Tag>(p, softcap, grid, stream);

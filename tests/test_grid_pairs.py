@@ -50,6 +50,17 @@ int main() {
       if (r < 0 || r >= n || seen[r]++) return std::printf("rank %d of %d -> %d\n", k, n, r), 1;
     }
   }
+  // head_dim 32 only where pairing is faster: with softcap past 384 workgroups
+  for (int d : {8, 16, 32}) {
+    if (ffa::prefill_pairs(d, false, 512) || ffa::prefill_pairs(d, true, 384) ||
+        !ffa::prefill_pairs(d, true, 385)) {
+      return std::printf("head_dim %d\n", d), 1;
+    }
+  }
+  for (int d : {40, 64, 128, 192}) {
+    if (!ffa::prefill_pairs(d, false, 257)) return std::printf("head_dim %d\n", d), 1;
+  }
+  if (ffa::prefill_pairs(200, true, 400)) return std::printf("head_dim 200\n"), 1;
   std::printf("ok %d\n", paired);
   return paired == 0;
 }
