@@ -84,6 +84,17 @@ struct Shape {
 template <int DP, bool SOFTCAP>
 constexpr int kMinBlocks = (DP == 64 && !SOFTCAP) ? 3 : (DP <= 192 ? 2 : 1);
 
+// Whether a kernel holds the code of a block mask. Calls with one have kernels of their own
+// (Tag = BlockMask<...>): its tile list and the search for its fast runs took scalar registers
+// that the others then spilled (52 instead of 19 at head_dim 32 with softcap), which slowed
+// calls without a mask. On MI355X, B 2, 32/8 heads, S 2048, and B 1, 8/8 heads, S 7000, us in
+// one kernel / apart: D 32 softcap 53.3 / 52.6, 104.4 / 100.9; D 64 window 700 44.0 / 37.5, 30.8
+// / 23.7 (its tiles at the edges tested a mask bit per element); D 128 79.7 / 79.0, softcap and window 40.9 / 39.8; D 192 softcap and window 54.2 /
+// 52.7. One kernel for both where that is as fast (head_dim 256 with softcap 247.7 / 249.4), for
+// split keys, and for a narrow V, whose kernels have no fast runs.
+template <typename Tag, int DP, int DV, bool SOFTCAP>
+constexpr bool kHoldsMask = kBlockMask<Tag> || kSplitKeys<Tag> || DV < DP || (DP == 256 && SOFTCAP);
+
 // DV: the V tile / O accumulator width (<= DP). It is DP except for head_dim 192 over
 // a V of at most 128 dims (the MLA prefill's V, which its caller would otherwise
 // zero-pad to 192): P V then runs over the 128 real dims only.
@@ -205,7 +216,8 @@ __global__ __launch_bounds__((64 * NW), (kMinBlocks<DP, SOFTCAP> * 4 / NW)) void
   const int qwl_abs = pack ? ql_abs : q_offset + min(qw0 + 31, p.Sq - 1);
   const int qa = q_offset + qrow;
   // block mask: this lane's row block in the expanded key mask
-  const uint64_t* const kmask = p.kmask;  // (a split call has no cached keys with one)
+  constexpr bool MASK = kHoldsMask<Tag, DP, DV, SOFTCAP>;
+  const uint64_t* const kmask = MASK ? p.kmask : nullptr;  // (a split call has no cached keys with one)
   const uint64_t* kmask_row =
       kmask != nullptr ? kmask + static_cast<int64_t>(min(qrow, p.Sq - 1) / p.ref_bq) * p.kmask_words
                          : nullptr;
@@ -1016,11 +1028,21 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(const PrefillParams 
 
 template <typename Tag, int DP, int DV, int BN, int NW>
 void launch_nw(const PrefillParams& p, bool softcap, int grid, hipStream_t s) {
-  const size_t dyn = p.kmask != nullptr ? kLiveLdsBytes : 0;
+  auto run = [&](auto cap) {
+    constexpr bool CAP = decltype(cap)::value;
+    if (p.kmask == nullptr) {
+      hipLaunchKernelGGL((prefill_kernel<Tag, DP, DV, BN, CAP, NW>), dim3(grid), dim3(64 * NW), 0, s, p);
+    } else if constexpr (kHoldsMask<Tag, DP, DV, CAP>) {
+      hipLaunchKernelGGL((prefill_kernel<Tag, DP, DV, BN, CAP, NW>), dim3(grid), dim3(64 * NW), kLiveLdsBytes, s, p);
+    } else {
+      hipLaunchKernelGGL((prefill_kernel<BlockMask<Tag>, DP, DV, BN, CAP, NW>), dim3(grid), dim3(64 * NW),
+                         kLiveLdsBytes, s, p);
+    }
+  };
   if (softcap) {
-    hipLaunchKernelGGL((prefill_kernel<Tag, DP, DV, BN, true, NW>), dim3(grid), dim3(64 * NW), dyn, s, p);
+    run(std::true_type{});
   } else {
-    hipLaunchKernelGGL((prefill_kernel<Tag, DP, DV, BN, false, NW>), dim3(grid), dim3(64 * NW), dyn, s, p);
+    run(std::false_type{});
   }
 }
 

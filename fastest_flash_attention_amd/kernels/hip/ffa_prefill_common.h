@@ -17,6 +17,16 @@ constexpr bool kSplitKeys = false;
 template <typename Tag>
 constexpr bool kSplitKeys<SplitKeys<Tag>> = true;
 
+// Marks the element tag of a kernel compiled for launches with a block mask.
+template <typename Tag>
+struct BlockMask {};
+template <typename Tag>
+struct Elem<BlockMask<Tag>> : Elem<Tag> {};
+template <typename Tag>
+constexpr bool kBlockMask = false;
+template <typename Tag>
+constexpr bool kBlockMask<BlockMask<Tag>> = true;
+
 namespace pf {
 
 constexpr float kRescaleThresh = 8.0f;  // log2 units: the running max moves only past this

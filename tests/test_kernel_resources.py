@@ -36,7 +36,8 @@ EXCEPTIONS = {
 }
 
 
-def _scratch_by_kernel(src: str, tmp: str) -> dict:
+def _spills_by_kernel(src: str, tmp: str) -> dict:
+    """Kernel name -> (scratch bytes per lane, scalar registers spilled to vector lanes)."""
     out = os.path.join(tmp, os.path.basename(src) + ".s")
     cmd = [build.hipcc(), *build.HIPCC_FLAGS, f"-I{build.INCLUDE}", f"-I{build.HERE}",
            "--cuda-device-only", "-S", src, "-o", out]
@@ -46,8 +47,8 @@ def _scratch_by_kernel(src: str, tmp: str) -> dict:
     res = {}
     for block in text.split("\n  - .agpr_count:")[1:]:
         name = re.search(r"\.name:\s+(\S+)", block).group(1)
-        priv = int(re.search(r"\.private_segment_fixed_size:\s+(\d+)", block).group(1))
-        res[name] = priv
+        res[name] = tuple(int(re.search(rf"\.{key}:\s+(\d+)", block).group(1))
+                          for key in ("private_segment_fixed_size", "sgpr_spill_count"))
     return res
 
 
@@ -59,14 +60,20 @@ def _demangle(names):
     return dict(zip(names, r.stdout.splitlines()))
 
 
-@pytest.mark.skipif(shutil.which("hipcc") is None and not os.path.exists("/opt/rocm/bin/hipcc"),
-                    reason="hipcc not installed")
-def test_hot_kernels_do_not_spill(tmp_path):
+@pytest.fixture(scope="module")
+def spills(tmp_path_factory):
+    if shutil.which("hipcc") is None and not os.path.exists("/opt/rocm/bin/hipcc"):
+        pytest.skip("hipcc not installed")
+    tmp = str(tmp_path_factory.mktemp("asm"))
     srcs = [os.path.join(build.HERE, f) for f in
             ("ffa_prefill.hip", "ffa_decode.hip", "ffa_backward.hip")]
     with ThreadPoolExecutor(3) as ex:
-        parts = list(ex.map(lambda s: _scratch_by_kernel(s, str(tmp_path)), srcs))
-    scratch = {k: v for part in parts for k, v in part.items()}
+        parts = list(ex.map(lambda s: _spills_by_kernel(s, tmp), srcs))
+    return {k: v for part in parts for k, v in part.items()}
+
+
+def test_hot_kernels_do_not_spill(spills):
+    scratch = {k: v[0] for k, v in spills.items()}
     assert len(scratch) >= 60, f"only {len(scratch)} kernels found"
     names = _demangle(list(scratch))
     bad = []
@@ -82,3 +89,19 @@ def test_hot_kernels_do_not_spill(tmp_path):
     # the headline kernel in particular
     ns = [n for m, n in names.items() if re.search(r"prefill_kernel<ffa::Bf16Tag, 128, 128, 64, false, 4>", n)]
     assert ns and all(scratch[m] == 0 for m, n in names.items() if n in ns)
+
+
+def test_kernels_without_a_block_mask_spare_its_registers(spills):
+    """Calls without a block mask run kernels without its code: the list of tiles and its fast
+    runs take scalar registers, and where one kernel held both the loops of every call reloaded
+    up to 52 of them. (Bound: half of what one kernel for both spills.)"""
+    names = _demangle(list(spills))
+    by_name = {n: spills[m][1] for m, n in names.items()}
+    pairs = 0
+    for name, masked in by_name.items():
+        if "BlockMask<" not in name:
+            continue
+        plain = by_name[re.sub(r"ffa::BlockMask<(ffa::\w+)>", r"\1", name)]
+        assert 2 * plain <= masked, f"{name}: {masked} scalar spills, without a mask {plain}"
+        pairs += 1
+    assert pairs >= 18
