@@ -218,6 +218,10 @@ __global__ __launch_bounds__((64 * NW), (kMinBlocks<DP, SOFTCAP> * 4 / NW)) void
   // block mask: this lane's row block in the expanded key mask
   constexpr bool MASK = kHoldsMask<Tag, DP, DV, SOFTCAP>;
   const uint64_t* const kmask = MASK ? p.kmask : nullptr;  // (a split call has no cached keys with one)
+  // (drops the fast range of calls without one: with it the loops of these kernels reload up
+  // to 55 scalar registers instead of 36, masks without runs 187 / 179 us at D 192 with
+  // softcap, 251 / 242 at D 256, 316 / 308 at D 64 with softcap)
+  if constexpr (kBlockMask<Tag>) __builtin_assume(kmask != nullptr);
   const uint64_t* kmask_row =
       kmask != nullptr ? kmask + static_cast<int64_t>(min(qrow, p.Sq - 1) / p.ref_bq) * p.kmask_words
                          : nullptr;
@@ -828,10 +832,11 @@ __global__ __launch_bounds__((64 * NW), (kMinBlocks<DP, SOFTCAP> * 4 / NW)) void
   if (!NARROW && wave_live && use_list) {  // (the narrow-V kernels would spill)
     // Block mask: the first run of at least four list positions whose tiles are kept whole
     // and follow one another (the running tile pointers of the fast steps advance by one
-    // tile), and pass the tests above: the inside of a band or of a causal mask. On
-    // MI355X over 8000 tokens (B 2, 16 heads, D 128, causal): a local band of 19 live tiles
-    // a workgroup 210 -> 185 us, a causal mask 566 -> 474, random tiles (no run) 483 -> 487;
-    // the band at D 256 (B 1) 313 -> 228.
+    // tile), and pass the tests above: the inside of a band or of a causal mask. On MI355X
+    // over 8000 tokens (8 heads, D 128, causal, 64 x 64 tiles), us without / with fast runs: a
+    // band of 11 tiles a row 44.8 / 40.3, a causal mask 211 / 141, random tiles (no run) 314 /
+    // 303, six columns of tiles and the band 52.6 / 51.1, and a band of 41 110 / 110 (the first
+    // run is that of the columns); at D 256 113 / 89, 442 / 274, 505 / 492, 149 / 135, 335 / 319.
     int run = 0;  // length of the run that ends before position `base`
     for (int base = 0; base < n_it; base += 64) {
       const int j = base + lane;

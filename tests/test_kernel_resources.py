@@ -91,17 +91,25 @@ def test_hot_kernels_do_not_spill(spills):
     assert ns and all(scratch[m] == 0 for m, n in names.items() if n in ns)
 
 
-def test_kernels_without_a_block_mask_spare_its_registers(spills):
-    """Calls without a block mask run kernels without its code: the list of tiles and its fast
-    runs take scalar registers, and where one kernel held both the loops of every call reloaded
-    up to 52 of them. (Bound: half of what one kernel for both spills.)"""
+# padded head_dim -> scalar registers that one kernel for calls with and without a block mask
+# spilled before it searched the mask for fast runs; with the search up to 52 (head_dim 32) and
+# 55 (192), and calls of either kind were 1-4 % slower
+SCALAR_SPILLS = {32: 17, 64: 28, 128: 54, 192: 41, 256: 50}
+
+
+def test_block_masks_have_kernels_of_their_own(spills):
+    """Calls without a block mask run kernels without its code, and those with one kernels
+    without the code of the others: neither reloads more scalar registers in its loops than
+    one kernel for both did without fast runs."""
     names = _demangle(list(spills))
     by_name = {n: spills[m][1] for m, n in names.items()}
-    pairs = 0
+    found = 0
     for name, masked in by_name.items():
-        if "BlockMask<" not in name:
+        m = re.search(r"BlockMask<ffa::\w+>, (\d+), ", name)
+        if m is None:
             continue
         plain = by_name[re.sub(r"ffa::BlockMask<(ffa::\w+)>", r"\1", name)]
-        assert 2 * plain <= masked, f"{name}: {masked} scalar spills, without a mask {plain}"
-        pairs += 1
-    assert pairs >= 18
+        limit = SCALAR_SPILLS[int(m.group(1))]
+        assert plain <= limit and masked <= limit, f"{name}: {masked} scalar spills, without {plain}"
+        found += 1
+    assert found >= 18
