@@ -376,10 +376,6 @@ def dtype_code(dtype: torch.dtype, allow_fp32: bool = False) -> int:
     )
 
 
-def current_stream_handle(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
-
-
 def launch(fn, args: ctypes.Structure, device: torch.device) -> None:
     """Call an entry point on ``device``'s current stream with that device current; raise on
     a status other than FFA_OK. The stream is read as the raw handle and the device is

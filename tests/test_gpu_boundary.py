@@ -65,7 +65,7 @@ def test_abi_scale_contract(name, dtype, scale, softcap, causal):
                               softcap=softcap, return_lse=True)
     assert call.args.scale == np.float32(scale)  # the Python layer passes it unchanged
     lib = _lib.load()
-    stream = _lib.current_stream_handle(call.q.device)
+    stream = torch.cuda.current_stream(call.q.device).cuda_stream
     rc = lib.ffa_prefill_fwd(ctypes.byref(call.args), ctypes.c_void_p(stream))
     assert rc == 0, _lib.strerror(rc)
     torch.cuda.synchronize()
