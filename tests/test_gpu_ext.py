@@ -10,6 +10,7 @@ import pytest
 import torch
 
 import fastest_flash_attention_amd as ffa
+from fastest_flash_attention_amd.ops.attention_forward import prepare_prefill
 from oracle import reference_forward as rf
 from tests.gpu_util import assert_parity, np32, require_gpu, say, seeded
 
@@ -117,8 +118,9 @@ def test_block_mask_tile_skipping_parity(case):
 
 
 def test_block_mask_long_sweep_visits_every_tile():
-    """A sweep longer than the live-tile list (2048 tiles of 64 keys) visits every tile;
-    an all-true mask there still equals the unmasked result bit for bit."""
+    """A mask over more keys than one live-tile list holds (2048 tiles of 64), in a call whose
+    keys are split: every range lists its own tiles, and an all-true mask still equals the
+    unmasked result bit for bit. (Unsplit sweeps past the list: tests/test_split.py.)"""
     require_gpu()
     Skv = 2048 * 64 + 1000
     q = seeded((1, 1, 48, 64), BF16, 51).cuda()
@@ -127,6 +129,7 @@ def test_block_mask_long_sweep_visits_every_tile():
     say(f"block_mask long sweep Skv{Skv}")
     dense, dl = ffa.fastest_flash_attn_forward(q, k, v, block_size=64, return_lse=True)
     full = torch.ones(1, math.ceil(Skv / 64), dtype=torch.bool)
+    assert prepare_prefill(q, k, v, block_size=64, block_mask=full).args.workspace
     masked, ml = ffa.fastest_flash_attn_forward(q, k, v, block_size=64, block_mask=full,
                                                 return_lse=True)
     assert torch.equal(dense, masked) and torch.equal(dl, ml)

@@ -15,7 +15,7 @@ SOURCE = r"""
 #include "ffa_grid.h"
 
 int main() {
-  int paired = 0;
+  int paired = 0, lighter = 0;
   for (int units = 1; units <= 64; ++units) {
     for (int n_t = 1; n_t <= 64; ++n_t) {
       const int grid = units * n_t;
@@ -38,9 +38,12 @@ int main() {
         ffa::prefill_work_item(bid, grid, n_t, group & (ffa::kPaired - 1), remap, u, j);
         plain[c] += n_t - j;
       }
-      if (*std::max_element(cu.begin(), cu.end()) > *std::max_element(plain.begin(), plain.end())) {
-        return std::printf("units %d tiles %d: heavier than unpaired\n", units, n_t), 1;
-      }
+      const long most = *std::max_element(cu.begin(), cu.end());
+      const long before = *std::max_element(plain.begin(), plain.end());
+      if (most > before) return std::printf("units %d tiles %d: heavier than unpaired\n", units, n_t), 1;
+      lighter += most < before;
+      // a full launch: every CU gets the two tiles whose weights add up to n_t + 1
+      if (grid == 512 && most > n_t + 1) return std::printf("units %d tiles %d: %ld\n", units, n_t, most), 1;
     }
   }
   for (int n = 257; n <= 512; ++n) {
@@ -61,8 +64,8 @@ int main() {
     if (!ffa::prefill_pairs(d, false, 257)) return std::printf("head_dim %d\n", d), 1;
   }
   if (ffa::prefill_pairs(200, true, 400)) return std::printf("head_dim 200\n"), 1;
-  std::printf("ok %d\n", paired);
-  return paired == 0;
+  std::printf("ok %d, %d of them lighter\n", paired, lighter);
+  return paired == 0 || 2 * lighter < paired;
 }
 """
 

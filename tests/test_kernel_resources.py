@@ -1,5 +1,5 @@
-"""Register-spill guard (CPU, no GPU needed): compile the prefill, decode and backward
-translation units for gfx950 with the library's own flags and read every kernel's
+"""Register-spill guard (CPU, no GPU needed): compile the library's kernel translation units
+for gfx950 with the library's own flags and read every kernel's
 private-segment (scratch) size from the code-object metadata.
 
 Scratch reloads inside a kernel's KV loop come with `s_waitcnt vmcnt` waits that also
@@ -65,8 +65,7 @@ def spills(tmp_path_factory):
     if shutil.which("hipcc") is None and not os.path.exists("/opt/rocm/bin/hipcc"):
         pytest.skip("hipcc not installed")
     tmp = str(tmp_path_factory.mktemp("asm"))
-    srcs = [os.path.join(build.HERE, f) for f in
-            ("ffa_prefill.hip", "ffa_decode.hip", "ffa_backward.hip")]
+    srcs = [os.path.join(build.HERE, f) for f in build.SOURCES if f != "ffa_api.hip"]
     with ThreadPoolExecutor(3) as ex:
         parts = list(ex.map(lambda s: _spills_by_kernel(s, tmp), srcs))
     return {k: v for part in parts for k, v in part.items()}

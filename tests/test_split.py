@@ -342,10 +342,12 @@ def test_split_calls_under_capture_and_on_two_streams():
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("name", ["band", "runs", "causal"])
-@pytest.mark.parametrize("D,softcap", [(128, None), (64, 20.0)])
+@pytest.mark.parametrize("D,softcap", [(128, None), (64, 20.0), (32, None), (64, None), (192, None),
+                                       (192, 20.0), (256, None), (256, 20.0)])
 def test_block_mask_runs(name, D, softcap):
     """Runs of whole, consecutive tiles in the live-tile list take the fast steps: runs that
-    start at odd positions, end inside and cross the 64 positions looked at together."""
+    start at odd positions, end inside and cross the 64 positions looked at together (128 of
+    32 keys from head_dim 192 on)."""
     require_gpu()
     S, Hq, n = 4400, 4, 69  # 140 workgroups: not split
     bm = torch.zeros(n, n, dtype=torch.bool)
@@ -376,3 +378,59 @@ def test_block_mask_runs(name, D, softcap):
             softcap=softcap, sliding_window=None, two_pass=False, compute_dtype=None, q_offset=off,
             return_lse=True)
         assert_parity(o[:, :, a:b], ro, lse[:, :, a:b], rl, f"{name} tile {t}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,softcap", [(64, None), (128, 20.0), (128, None), (192, None), (192, 20.0),
+                                       (256, None), (256, 20.0)])
+@pytest.mark.parametrize("causal", [False, True])
+def test_split_block_mask_runs(D, softcap, causal):
+    """The same in split calls, whose ranges have lists of their own: whole tiles on both sides
+    of a range's end, holes inside ranges, and a run up to the ragged last tile."""
+    require_gpu()
+    Hq, Sq, Skv = (2, 2500, 2500) if causal else (4, 300, 9017)
+    say(f"split mask runs D{D} cap{softcap} causal{causal}")
+    q = seeded((1, Hq, Sq, D), BF16, 1)
+    k, v = (seeded((1, 1, Skv, D), BF16, s) for s in (2, 3))
+    bm = torch.ones(math.ceil(Sq / 64), math.ceil(Skv / 64), dtype=torch.bool)
+    bm[:, 13] = bm[:, 30:32] = False
+    bm[1::2, 21] = False
+    kw = dict(causal=causal, num_kv_heads=1, softcap=softcap, block_size=64)
+    args = (q.cuda(), k.cuda(), v.cuda())
+    assert af.prepare_prefill(*args, block_mask=bm, **kw).args.workspace  # split
+    o, lse = ffa.fastest_flash_attn_forward(*args, block_mask=bm, return_lse=True, **kw)
+    ro, rl = rf.forward(np32(q), np32(k), np32(v), block_mask=bm.numpy(), return_lse=True, **kw)
+    assert_parity(o, ro, lse, rl, "split mask runs")
+
+
+def _broadcast(t, dim):
+    """t's first entry along dim, repeated without a copy, and the same values in memory."""
+    one = t.narrow(dim, 0, 1)
+    wide = one.expand(t.shape)
+    return (one if dim == 0 else wide), wide.contiguous()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dim", [0, 1], ids=["batch", "heads"])
+@pytest.mark.parametrize("Sq,Sc", [(1, 900), (5, 700), (130, 333), (40, 0)])
+def test_broadcast_keys_are_read_in_place(dim, Sq, Sc):
+    """One batch entry of k, v and the cache under a larger batch of queries, and one head
+    expanded to all: read through zero strides, the same bits as from memory."""
+    require_gpu()
+    B, Hq, Hkv, D = 3, 8, 4, 128
+    say(f"split broadcast dim{dim} Sq{Sq} Sc{Sc}")
+    q = seeded((B, Hq, Sq, D), BF16, 1).cuda()
+    own = Sq if Sc else 2300
+    pairs = [_broadcast(seeded((B, Hkv, n, D), BF16, s).cuda(), dim)
+             for n, s in ((own, 2), (own, 3), (max(Sc, 1), 4), (max(Sc, 1), 5))]
+    outs = []
+    for form in (0, 1):
+        k, v, kc, vc = (p[form] for p in pairs)
+        kw = dict(causal=bool(Sc), num_kv_heads=Hkv, kv_cache=(kc, vc) if Sc else None)
+        args = af.prepare_prefill(q, k, v, **kw).args
+        assert args.workspace and bool(args.k_cache) == bool(Sc)  # split, the cache in place
+        outs.append(ffa.fastest_flash_attn_forward(q, k, v, return_lse=True, **kw))
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+    ro, rl = rf.forward(np32(q), np32(k), np32(v), return_lse=True, causal=bool(Sc),
+                        num_kv_heads=Hkv, kv_cache=(np32(kc), np32(vc)) if Sc else None)
+    assert_parity(outs[0][0], ro, outs[0][1], rl, "broadcast")
