@@ -664,9 +664,9 @@ __global__ __launch_bounds__(kThreads, kBwdMinBlocks<DP>) void bwd_dkdv_kernel(c
 }
 
 // dK and dV of the key tiles whose sweep was cut: the sum of its parts in part order.
-// One thread per 4 dims of a key; grid (cut key tile, part of its rows). Bound by HBM: 13 us on
-// MI355X at B 2, 32/8 heads, S 2011, D 128 (three parts at most, 4 TB/s), beside 200 us of
-// the cut kernel and 317 of the uncut one.
+// One thread per 4 dims of a key; grid (cut key tile, part of its rows). Bound by HBM: 11 us on
+// MI355X at B 2, 32/8 heads, S 2011, D 128 (three parts at most), beside 197 us of the cut
+// kernel and 317 of the uncut one.
 template <typename Tag>
 __global__ __launch_bounds__(kThreads) void bwd_dkdv_sum_kernel(const BwdParams p) {
   using E = Elem<Tag>;

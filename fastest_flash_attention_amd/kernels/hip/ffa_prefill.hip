@@ -426,8 +426,8 @@ __global__ __launch_bounds__((64 * NW), (kMinBlocks<DP, SOFTCAP> * 4 / NW)) void
   // where S^T(t+1) is a block of 24-32 MFMAs ahead of softmax(t)) the compiler spreads
   // the tile's max and softcap VALU work of tile t between those MFMAs: +2 % at the MLA
   // prefill shape, +5-6 % at head_dim 192 with softcap and at 256 on MI355X,
-  // bit-identical (two head_dim-192 kernels then use 12 B per lane of scratch, reloaded in
-  // the general-step loops, not in the fast loop; still faster).
+  // bit-identical (the four-wave narrow-V kernel then uses 8 B per lane of scratch, reloaded
+  // in the general-step loops, not in the fast loop; still faster).
   auto qk = [&](const uint16_t* kl, f32x16 (&sacc)[S::NB], auto fence) __attribute__((always_inline)) {
     constexpr bool FENCE = decltype(fence)::value;
 #pragma unroll
